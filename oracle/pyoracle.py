@@ -49,9 +49,9 @@ _i32p = ctypes.POINTER(ctypes.c_int32)
 
 
 def build() -> None:
-    """Compile liboracle.so (and oracle/_ref when the reference is present)."""
+    """Compile liboracle.so (and oracle/_ref when the reference's sources are present)."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isdir("/root/reference/StandAlone"):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
