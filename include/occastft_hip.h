@@ -144,7 +144,7 @@ void ostft_destroy(ostft_ctx* ctx);
  * aligned) are device pointers on the context's device; work is queued on `hip_stream`
  * (a hipStream_t, or NULL for the null stream) and this call does not wait
  * for it.  The first call for a new (window, exp) builds the window and
- * FP64-generated twiddle tables synchronously.  Windows 2^16..2^20 pass
+ * FP64-generated twiddle tables synchronously.  Windows 2^17..2^20 pass
  * through the context's scratch buffer: a call on another stream than the
  * previous such call first makes its stream wait for that call's launches.
  * Replaces the device part of Runner::ActivateSTFT. */
@@ -159,20 +159,20 @@ int ostft_run_device(ostft_ctx* ctx, const ostft_params* params, const float* d_
  *     in the context (one ostft_run_device or ostft_activate call with the
  *     same window kind, size and sigma builds them); otherwise the call
  *     returns OSTFT_ERR_NOT_PREPARED and launches nothing;
- *   - windows 2^16..2^20 pass their intermediate spectra through a fixed
+ *   - windows 2^17..2^20 pass their intermediate spectra through a fixed
  *     64 MiB device array per GPU (frames in chunks of 64 MiB / (4 N) bytes:
  *     16 frames at 2^20) instead of the context's growable scratch, with no
  *     event.  Every call on a GPU shares that array and it keeps the last
  *     call's contents (each call overwrites what it reads first): calls that
  *     overlap in time on one GPU race; keep them on one stream or ordered.
- * Windows up to 2^15 use no scratch. */
+ * Windows up to 2^16 use no scratch. */
 int ostft_run_device_noalloc(ostft_ctx* ctx, const ostft_params* params, const float* d_in,
                              uint64_t full_size, float* d_out, uint64_t out_cap, void* hip_stream);
 
 /* Strided batch of `count` equal requests: signal y is d_in + y * in_stride
  * (full_size floats), its result goes to d_out + y * out_stride (out_stride a
  * multiple of 4 floats, at least the layout's out_floats).  One launch (for
- * windows up to 2^15); results are bitwise those of ostft_run_device on each
+ * windows up to 2^16); results are bitwise those of ostft_run_device on each
  * signal.  No counterpart in the reference (one signal per ActivateSTFT). */
 int ostft_run_strided_device(ostft_ctx* ctx, const ostft_params* params, const float* d_in,
                              uint64_t full_size, uint64_t in_stride, uint32_t count, float* d_out,
@@ -260,7 +260,7 @@ int ostft_engine_variant(ostft_ctx* ctx, int32_t exp, int32_t shape, int32_t pla
 int ostft_autotune_batch(ostft_ctx* ctx, int32_t exp, uint64_t samples, const ostft_params* like,
                          int32_t* best_blocks_per_cu, int32_t* best_shape, int32_t* best_plan, double* best_ms);
 
-/* Scratch budget of the two-pass path (windows 2^16..2^20), in bytes: its
+/* Scratch budget of the two-pass path (windows 2^17..2^20), in bytes: its
  * frames go through both passes in chunks whose intermediate spectra fit the
  * budget (at least one frame per chunk).  bytes = 0 leaves it; a budget below
  * the scratch already held frees that scratch.  *current (may be NULL)

@@ -11,7 +11,7 @@
 // block, so for a given set of classes they are the same every time: they are
 // captured once into a HIP graph and replayed.
 //
-// Requests of windows >= 2^16 (multi-pass path) and requests of the matrix-core
+// Requests of windows >= 2^16 (one launch, or the two-pass path) and requests of the matrix-core
 // form run after the tile-queue launches, one request at a time, on the same
 // stream.
 #include <hip/hip_runtime.h>
@@ -425,6 +425,12 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
             return ctx_hip_fail(ctx, e, "batch MFMA launch");
     }
     for (uint32_t i : large) {
+        if (wide_supported(lm[i])) {
+            const hipError_t e = launch_wide(args[i], 1, s);
+            if (e != hipSuccess)
+                return ctx_hip_fail(ctx, e, "batch wide launch");
+            continue;
+        }
         rc = run_multipass(ctx, lm[i], args[i], s);
         if (rc != OSTFT_OK)
             return rc;

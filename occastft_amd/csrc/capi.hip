@@ -426,7 +426,7 @@ int ctx_prepare(ostft_ctx* ctx, const ostft_params* params, const float* d_in, u
     a->tw_n = get_twiddles(ctx, 2 * M, M, &rc, noalloc);  // W_N^k, k < M
     if (!a->tw_n)
         return rc;
-    if (fused_supported(plan.log_m)) {
+    if (fused_supported(plan.log_m) || wide_supported(plan.log_m)) {
         a->tw = get_twiddles(ctx, M, M, &rc, noalloc);
         if (!a->tw)
             return rc;
@@ -646,6 +646,10 @@ int run_device_geometry(ostft_ctx* ctx, const ostft_params* params, const float*
             return hip_fail(ctx, e, "fused STFT launch");
         return OSTFT_OK;
     }
+    if (ostft::wide_supported(log_m)) {
+        const hipError_t e = ostft::launch_wide(a, 1, s);
+        return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "wide STFT launch");
+    }
     return ostft::run_multipass(ctx, log_m, a, s);
 }
 }  // namespace
@@ -684,6 +688,10 @@ int ostft_run_device_noalloc(ostft_ctx* ctx, const ostft_params* params, const f
         hipError_t e = ostft::launch_fused(log_m, transform_of(params), a, 1, s);
         return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "fused STFT launch");
     }
+    if (ostft::wide_supported(log_m)) {
+        const hipError_t e = ostft::launch_wide(a, 1, s);
+        return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "wide STFT launch");
+    }
     return ostft::run_multipass_static(ctx, ctx->device, log_m, a, s);
 }
 
@@ -710,12 +718,14 @@ int ostft_run_strided_device(ostft_ctx* ctx, const ostft_params* params, const f
         return OSTFT_OK;
     a.in_stride = in_stride;
     a.out_stride = out_stride;
-    if (ostft::fused_supported(log_m)) {
+    if (ostft::fused_supported(log_m) || ostft::wide_supported(log_m)) {
         for (uint32_t y0 = 0; y0 < count; y0 += 65535u) {  // grid.y limit
             ostft::FusedArgs ay = a;
             ay.in = d_in + (uint64_t)y0 * in_stride;
             ay.out = d_out + (uint64_t)y0 * out_stride;
-            const hipError_t e = ostft::launch_fused(log_m, transform_of(params), ay, std::min(count - y0, 65535u), s);
+            const uint32_t n = std::min(count - y0, 65535u);
+            const hipError_t e = ostft::wide_supported(log_m) ? ostft::launch_wide(ay, n, s)
+                                                              : ostft::launch_fused(log_m, transform_of(params), ay, n, s);
             if (e != hipSuccess)
                 return hip_fail(ctx, e, "strided STFT launch");
         }

@@ -1,5 +1,5 @@
 // engine.hpp -- internal interface between the C ABI (capi.hip) and the
-// kernels (fused_small.hip, tables.hip, multipass.hip).
+// kernels (fused_small.hip, fused_wide.hip, tables.hip, multipass.hip).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -74,6 +74,11 @@ int fused_variant_frames(int log_m, int variant);
 bool fused_plan_ok(int log_m, int plan);
 // `count` signals (grid.y), signal y at a.in + y in_stride / a.out + y out_stride
 hipError_t launch_fused(int log_m, int xf, const FusedArgs& a, uint32_t count, hipStream_t s);
+
+// One workgroup per frame with the transform in registers (fused_wide.hip):
+// complex size 2^15 (window 2^16).
+bool wide_supported(int log_m);
+hipError_t launch_wide(const FusedArgs& a, uint32_t count, hipStream_t s);
 
 // ---- batches: many requests of one window size in one persistent launch ----
 // A batch descriptor block lives in device memory (uploaded by the host before

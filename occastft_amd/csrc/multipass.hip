@@ -1,6 +1,5 @@
-// multipass.hip -- STFT for complex transform sizes M = 2^15 .. 2^19
-// (windows 2^16 .. 2^20; the plan also covers M = 2^13, 2^14, which the
-// single kernel handles).
+// multipass.hip -- STFT for complex transform sizes M = 2^16 .. 2^19
+// (windows 2^17 .. 2^20).
 //
 // Same pipeline as the fused kernel (gather + window, FFT, split epilogue),
 // but the transform no longer fits one workgroup's LDS, so it is cut into two
@@ -382,9 +381,9 @@ int multipass_plan(int log_m, int* lr)
     // (R1 = 2^6: 256-byte runs of the real layouts; 2^8 gave 64-byte runs and
     // a 4-5% slower large-window step, 2^9 was 1.7x slower), the first radix
     // at most 2^11 (its column segments are CB = 8192 / R0 values)
-    if (log_m < 13 || log_m > 19)
+    if (log_m < 16 || log_m > 19)
         return 0;
-    lr[1] = log_m / 2 > 6 ? 6 : log_m / 2;
+    lr[1] = 6;
     if (log_m - lr[1] > 11)
         lr[1] = log_m - 11;
     lr[0] = log_m - lr[1];
@@ -414,9 +413,6 @@ static hipError_t launch_last(const LastArgs& p, hipStream_t s)
 static hipError_t first_pass(int log_r, const PassArgs& p, hipStream_t s)
 {
     switch (log_r) {
-    case 7: return launch_first<7>(p, s);
-    case 8: return launch_first<8>(p, s);
-    case 9: return launch_first<9>(p, s);
     case 10: return launch_first<10>(p, s);
     case 11: return launch_first<11>(p, s);
     default: return hipErrorInvalidValue;
@@ -563,7 +559,7 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     // allocation stays bounded (1 GiB by default) whatever the signal
     // length.  Chunks small enough for their scratch to stay in the 256 MB
     // memory-side cache between the passes measured slower (64 MiB: +15%,
-    // 128 MiB: +3% on windows 2^16..2^20): the passes are not bound by the
+    // 128 MiB: +3% on windows 2^16..2^20 when all of them came this way): the passes are not bound by the
     // round trip's HBM traffic, and every chunk adds two launch tails.
     const uint64_t chunk = even_chunk(a.frames, multipass_chunk_frames(sc.budget, log_m));
     hipError_t e = sc.ensure((a.frames < chunk ? a.frames : chunk) * M);

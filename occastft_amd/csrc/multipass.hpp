@@ -1,4 +1,4 @@
-// multipass.hpp -- large-window path (complex transform sizes 2^13 .. 2^19).
+// multipass.hpp -- large-window path (complex transform sizes 2^16 .. 2^19).
 #pragma once
 
 #include <mutex>
@@ -47,7 +47,7 @@ uint64_t multipass_static_scratch_bytes();
 // as many as fit `budget` bytes of scratch, at least one.
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m);
 
-// Radix split of 2^log_m into the two passes (returns 2; 0 outside 13..19).
+// Radix split of 2^log_m into the two passes (returns 2; 0 outside 16..19).
 int multipass_plan(int log_m, int* log_radix /* [4] */);
 
 }  // namespace ostft
