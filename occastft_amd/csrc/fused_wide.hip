@@ -18,6 +18,7 @@
 // 4.4 without the transforms, 3.8 without the exchanges, 4.0 without the
 // stores.  A persistent grid that loads the next frame while this one's result
 // goes out took 850 us (a wave's loads wait for the stores issued before them).
+#include "buffer.hpp"
 #include "engine.hpp"
 #include "epilogue.hpp"
 #include "stockham.hpp"
@@ -30,29 +31,6 @@ namespace {
 constexpr int WIDE_LOG_M = 15, WIDE_M = 1 << WIDE_LOG_M, WIDE_T = WIDE_M / 32;
 constexpr int WIDE_LDS = WIDE_M + WIDE_M / 32;  // floats of the exchange: one pad per 32
 static_assert(WIDE_LDS >= WIDE_M + 2, "the mirror exchange's M/2 + 1 complex values");
-
-// A buffer descriptor over `bytes` bytes from a wave-uniform address: a load
-// or store then takes one 32-bit lane offset and a scalar offset, where the
-// 64-bit addresses of 32 loads would cost two vector instructions each.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void* p, uint32_t bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
-}
-
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ float2 load2(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off)
-{
-    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0));
-}
-__device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off, float v)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, lane_off, off, 0);
-}
-__device__ __forceinline__ void store2(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off, float2 v)
-{
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, lane_off, off, 0);
-}
 
 // One component of an exchange between radix-32 passes: value q of the thread
 // goes to wr[QSTEP q], value m comes from rd[m (M/32 padded)].  The caller's
@@ -147,15 +125,15 @@ __device__ __forceinline__ void wide_frame(const FusedArgs& a, const float* __re
 
     // ---- last radix-2 stage and output: bin k gives positions k and M + k, and
     //      by the conjugate symmetry of a real frame's spectrum M - k and N - k ----
-    auto epilogue = [&](auto mode_c) {
+    auto epilogue = [&](auto mode_c, auto cut_c) {
         constexpr int MODE = decltype(mode_c)::value;
+        constexpr bool CUT = decltype(cut_c)::value;  // HALF_COMPLEX: the frame that out_limit cuts short
         constexpr bool HALF = MODE == OUT_POWER || MODE == OUT_HALF_SPECTRUM;
         constexpr bool CPLX = MODE == OUT_HALF_COMPLEX || MODE == OUT_HALF_SPECTRUM;
         constexpr int B = CPLX ? 8 : 4;                      // bytes of an output value
         constexpr int W = HALF ? M + 1 : N;                  // values of a frame
         const uint64_t base = f * (uint64_t)W;
         const auto bo = buffer(reinterpret_cast<char*>(out) + B * base, B * W);
-        // HALF_COMPLEX ends at out_limit, which cuts the last frame short
         const uint64_t room = a.out_limit > base ? a.out_limit - base : 0;
         auto put = [&](uint32_t lane, uint32_t pos, float2 x2, bool conj) {  // value at position lane + pos
             if constexpr (MODE == OUT_COMPAT_POWER)
@@ -164,7 +142,7 @@ __device__ __forceinline__ void wide_frame(const FusedArgs& a, const float* __re
                 store1(bo, B * lane, B * pos, magnitude(x2));
             else if constexpr (MODE == OUT_POWER)
                 store1(bo, B * lane, B * pos, power_of(x2));
-            else if (MODE == OUT_HALF_SPECTRUM || lane + pos < room)
+            else if (!CUT || lane + pos < room)
                 store2(bo, B * lane, B * pos, conj ? conj_value_of(x2) : value_of(x2));
         };
         const float2* const zm = zu + M / 2 - t;
@@ -192,11 +170,16 @@ __device__ __forceinline__ void wide_frame(const FusedArgs& a, const float* __re
         }
     };
     switch (a.out_mode) {
-    case OUT_COMPAT_POWER: epilogue(std::integral_constant<int, OUT_COMPAT_POWER>{}); break;
-    case OUT_MAGNITUDE: epilogue(std::integral_constant<int, OUT_MAGNITUDE>{}); break;
-    case OUT_HALF_COMPLEX: epilogue(std::integral_constant<int, OUT_HALF_COMPLEX>{}); break;
-    case OUT_POWER: epilogue(std::integral_constant<int, OUT_POWER>{}); break;
-    case OUT_HALF_SPECTRUM: epilogue(std::integral_constant<int, OUT_HALF_SPECTRUM>{}); break;
+    case OUT_COMPAT_POWER: epilogue(std::integral_constant<int, OUT_COMPAT_POWER>{}, std::false_type{}); break;
+    case OUT_MAGNITUDE: epilogue(std::integral_constant<int, OUT_MAGNITUDE>{}, std::false_type{}); break;
+    case OUT_HALF_COMPLEX:
+        if ((f + 1) * N <= a.out_limit)
+            epilogue(std::integral_constant<int, OUT_HALF_COMPLEX>{}, std::false_type{});
+        else
+            epilogue(std::integral_constant<int, OUT_HALF_COMPLEX>{}, std::true_type{});
+        break;
+    case OUT_POWER: epilogue(std::integral_constant<int, OUT_POWER>{}, std::false_type{}); break;
+    case OUT_HALF_SPECTRUM: epilogue(std::integral_constant<int, OUT_HALF_SPECTRUM>{}, std::false_type{}); break;
     default: break;
     }
 }

@@ -2,37 +2,50 @@
 // (windows 2^17 .. 2^20).
 //
 // Same pipeline as the fused kernel (gather + window, FFT, split epilogue),
-// but the transform no longer fits one workgroup's LDS, so it is cut into two
-// Stockham passes through HBM-resident scratch (this replaces the EXP
-// separate radix-2 StockHamCommon launches of OKL/EXPCommon.okl:194-245, one
-// per stage, and the separate ToPower / toHalfComplexFormat passes).
+// but the transform fits no workgroup's registers, so it is cut into two
+// Stockham passes M = R0 x R1 through HBM-resident scratch (this replaces the
+// EXP separate radix-2 StockHamCommon launches of OKL/EXPCommon.okl:194-245,
+// one per stage, and the separate ToPower / toHalfComplexFormat passes).
 //
-// Both passes work on 8192 complex values per workgroup (512 threads, 70 KB of
-// LDS): CB = 8192/R butterflies of one frame, gathered as R rows of CB
-// contiguous values (stride M/R), FFT'd as CB independent R-point transforms
-// with the fused kernel's LDS Stockham engine.
-//   * first pass (radix R0 <= 2^11): reads the signal itself (overlap gather +
-//     window), writes the Stockham outputs Y[g R0 + q] (each butterfly's R0
-//     results contiguous);
-//   * last pass (radix R1 <= 2^8, stride Ns = R0): applies the inter-pass
-//     twiddle W_M^{g m} from a two-level FP64 table, and holds a block of
-//     butterflies g together with its mirror block Ns - g (0 and Ns/2 are their
-//     own mirrors), so both Z[k] and Z[M-k] of every output index k are in its
-//     LDS: the split epilogue (last radix-2 stage, DC correction, output layout)
-//     runs there and the spectrum is written once.
+// Both passes hold 32 complex values a thread in registers, 16384 or 8192 a
+// workgroup, as R-point transforms of as many columns, and take a column in two
+// register steps of fused multiply-add butterflies (twisted_dft.hpp) with one
+// exchange between them, whose real and imaginary parts go through LDS in turn.
+//   * first pass (R0 = 2^10 = 32 x 32): samples come from the signal (overlap
+//     gather + window) straight into the registers of their butterfly, results
+//     leave from the registers;
+//   * last pass (R1 = 2^6 .. 2^9 = R1/16 x 16): the inter-pass twiddle is the
+//     twist of its butterflies and costs no products of its own.  A block of
+//     butterflies k is held together with its mirror block R0 - k (0 and R0/2
+//     are their own mirrors), so both Z[k] and Z[M-k] of every output index are
+//     at hand: the split epilogue (last radix-2 stage, DC correction, output
+//     layout) runs there and the spectrum is written once.
 // As in the fused kernel, a frame of N real samples is one complex transform
 // of M = N/2 points (even samples real, odd imaginary).  DC removal is applied
 // in the frequency domain: subtracting the frame mean only changes the k = 0
 // terms.
+//
+// Bound by memory traffic (signal, scratch twice, result): with the transforms
+// compiled out the passes took within 10% of their time.  Against the form before
+// (16 values a thread, samples and scratch staged through LDS on their way in
+// and out, 2 to 3 exchanges, VALU issue 41-72% of the time), 2^27 samples:
+// window 2^18, overlap 0, default layout 594 -> 507 us (2.15 GB moved, 4.2 TB/s; a
+// plain copy of 2 GiB runs at 4.9); 2^20, 75%, power 2050 -> 1590 us; 2^26
+// samples, 75%, default layout: 2^17 853 -> 839, 2^18 987 -> 878, 2^19 1040 -> 903,
+// 2^20 1239 -> 961 us; one frame: 20-26 -> 18-22 us.
 #include "../../include/occastft_hip.h"
 
+#include <algorithm>
+#include <iterator>
 #include <mutex>
 #include <string>
 
 #include "batch.hpp"
+#include "buffer.hpp"
 #include "epilogue.hpp"
 #include "multipass.hpp"
 #include "stockham.hpp"
+#include "twisted_dft.hpp"
 
 namespace ostft {
 
@@ -94,30 +107,20 @@ void Scratch::destroy()
     used = false;
 }
 
-// Extra complex values per LDS column: the workgroup's global <-> LDS
-// transposition writes one value per column across consecutive lanes, so an
-// odd column stride spreads those lanes over all banks (R + R/16 is a
-// multiple of 4: up to 16 lanes of a wave on one bank).
-// First pass: 16-byte loads of two neighbouring packed samples of a row
-// where the signal and the window allow it (half the load instructions).
-#ifndef OSTFT_MP_VEC4
-#define OSTFT_MP_VEC4 1
-#endif
-// First pass: its scratch rows written two values per 16-byte store.
-#ifndef OSTFT_MP_VEC4_ST
-#define OSTFT_MP_VEC4_ST 1
-#endif
-#ifndef OSTFT_MP_COL_PAD
-#define OSTFT_MP_COL_PAD 1
-#endif
+// The split M = R0 x R1: R0 = 2^10 = 32 x 32, R1 = 2^6 .. 2^9 = R1/16 x 16
+constexpr int MP_LOG_R0 = 10, MP_R0 = 1 << MP_LOG_R0;
+// Scratch of a frame is [g / 16][k][g mod 16] for butterfly g and result k of
+// the first pass: a run of 16 values is a cache line and a quarter wave.
+constexpr uint32_t MP_RUN = 16;
 
-// first pass: frames per workgroup-order group (see first_pass_kernel)
-#ifndef OSTFT_MP_FRAME_GROUP
-#define OSTFT_MP_FRAME_GROUP 1
-#endif
-
-constexpr int MP_THREADS = 512;
-constexpr int MP_ELEMS = 16 * MP_THREADS;  // complex values per workgroup
+// A workgroup's threads and complex values.  512 threads: two workgroups a CU
+// and longer runs in memory; 256 threads: twice the workgroups, for requests
+// that leave CUs idle otherwise.  A frame's arithmetic is the same in both.
+template <int THREADS>
+struct Tile {
+    static constexpr uint32_t ELEMS = 32 * THREADS;
+    static constexpr uint32_t LDS = ELEMS + ELEMS / 32;  // floats
+};
 
 struct PassArgs {
     const float* sig;  // first pass: the signal
@@ -125,309 +128,347 @@ struct PassArgs {
     uint64_t frame0, frames;  // frames [frame0, frames) of this launch; scratch row 0 = frame0
     const float* win;
     float2* dst;
-    const float2* tw_r;  // W_R^j, j < R
-    uint32_t log_m;
+    const float2* tw_r;  // W_R0^j, j < R0
 };
 
-template <int LOG_R>
-__global__ void __launch_bounds__(MP_THREADS) first_pass_kernel(const PassArgs a)
+// One component of the exchange between the two steps of R-point transforms of
+// a workgroup's C columns, r1 x R2 = R: row r of column c is staged at
+// r C + (r / r1) PAD + c.  Second-step butterfly g = t + T u (T threads a column
+// of U butterflies each) takes rows g + r1 m, value u + U m of the thread.
+template <int C, int R1STEP, int PAD, int T, int U, int COMP>
+__device__ __forceinline__ void gather_step(float2 (&v)[32], const float* rd)
 {
-    constexpr int R = 1 << LOG_R, CB = MP_ELEMS / R, T = R / 16, PADR = R + R / 16 + OSTFT_MP_COL_PAD;
-    static_assert(CB * T == MP_THREADS, "MP_THREADS threads per block");
-    __shared__ float2 lds[CB * PADR];
+    cfor<0, 32>([&](auto i) {
+        constexpr int I = decltype(i)::value, UU = I % U, MM = I / U;
+        const float x = rd[T * C * UU + (R1STEP * C + PAD) * MM];
+        if constexpr (COMP)
+            v[I].y = x;
+        else
+            v[I].x = x;
+    });
+}
 
-    const uint32_t tid = threadIdx.x;
-    const uint64_t M = 1ull << a.log_m;
-    const uint64_t bpg = M / MP_ELEMS;  // blocks per transform = (M / R) / CB
-    const uint64_t blk = xcd_block(blockIdx.x, gridDim.x);
-    // Workgroup order: frames in groups of FG; within a group, consecutive
-    // workgroups (one XCD, about the same time) take the GB blocks of a block
-    // group for each frame of the group in turn, then the next block group.
-    // The GB blocks share their 128-byte lines (a block's rows are CB values
-    // long), overlapping frames of a group share rows and the group shares
-    // each window segment, so those come from HBM about once per group; FG = 1
-    // is plain frame order.
-    constexpr uint32_t GB = CB >= 16 ? 1u : 16u / CB;  // bpg is a multiple of GB (M >= 2^13)
-    const uint64_t F = a.frames - a.frame0, fg = blk / (OSTFT_MP_FRAME_GROUP * bpg);
-    const uint64_t p0 = fg * OSTFT_MP_FRAME_GROUP;
-    if (p0 >= F)
-        return;  // uniform over the block
-    const uint64_t q = F - p0 < OSTFT_MP_FRAME_GROUP ? F - p0 : OSTFT_MP_FRAME_GROUP;  // frames in this group
-    const uint64_t i = blk - fg * OSTFT_MP_FRAME_GROUP * bpg, r = i % (q * GB);
-    const uint64_t P = a.frame0 + p0 + r / GB, bi = (i / (q * GB)) * GB + r % GB;
-    const uint32_t g0 = (uint32_t)bi * CB;
-    const uint32_t stride = (uint32_t)(M >> LOG_R);
-    PassTwiddles<LOG_R> tws;
-    load_pass_twiddles<LOG_R>(tws, a.tw_r, tid % T);
+// First pass: C = 16 (8 with 256 threads) butterflies g of one frame (columns),
+// lanes along the columns: the samples come straight into the butterflies'
+// registers and the results leave from them, in runs of C values either way.
+template <int LOG_M, int THREADS>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+    first_pass_kernel(const PassArgs a)
+{
+    constexpr uint32_t M = 1u << LOG_M, R = MP_R0, C = Tile<THREADS>::ELEMS / R, T = R / 32, STRIDE = M / R;
+    constexpr uint32_t PAD = C;           // spreads the 64 / C rows 32 t of a wave over the banks
+    constexpr uint32_t BPF = STRIDE / C;  // workgroups per frame
+    static_assert(MP_RUN % C == 0, "a workgroup's columns share their scratch runs");
+    __shared__ float lds[Tile<THREADS>::LDS];
+    static_assert(Tile<THREADS>::LDS >= Tile<THREADS>::ELEMS + PAD * (R / 32), "exchange");
 
-    // rows of CB contiguous packed samples z[n] = x[2n] + i x[2n+1], windowed
+    const uint32_t tid = threadIdx.x, c = tid % C, t = tid / C;
+    // plain workgroup order: an XCD (workgroup index mod 8) takes the same
+    // columns of every frame, so its L2 holds their part of the window (2^20:
+    // 512 KiB of 4 MiB); each XCD on frames of its own read it from beyond L2
+    // every time, 342 against 306 us a launch of 171 frames
+    const uint64_t P = a.frame0 + blockIdx.x / BPF;
+    const uint32_t g0 = (blockIdx.x % BPF) * C;
+
+    // packed samples z[n] = x[2n] + i x[2n+1], n = g + STRIDE (t + T j), windowed
+    float2 v[32];
     const uint64_t fs = P * a.hop;
-    const float2* win2 = reinterpret_cast<const float2*>(a.win);
-    const uint64_t n_last = g0 + (CB - 1) + (uint64_t)(R - 1) * stride;  // the block's last packed index
-    const bool inside = fs + 2 * n_last + 2 <= a.L;
-    if (OSTFT_MP_VEC4 && CB >= 2 && inside && (reinterpret_cast<uintptr_t>(a.sig + fs) & 15u) == 0 &&
-        (reinterpret_cast<uintptr_t>(win2) & 15u) == 0) {
-        // pairs of neighbouring packed samples (columns c, c + 1 of a row;
-        // n even, so each pair is one 16-byte block of signal and of window)
-        constexpr int CH = CB >= 2 ? CB / 2 : 1;
-        float4 xv[8], wv[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            const uint32_t n = g0 + 2u * (e % CH) + (e / CH) * stride;
-            xv[j] = *reinterpret_cast<const float4*>(a.sig + fs + 2ull * n);
-            wv[j] = win2 ? *reinterpret_cast<const float4*>(win2 + n) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    const uint32_t n0 = g0 + c + STRIDE * t;
+    constexpr uint32_t STEP = STRIDE * T;
+    const auto bw = buffer(a.win, a.win ? 8 * M : 0);
+    auto window = [&](auto sample) {
+        if (a.win) {
+            // of the window 16 values are in flight: the registers hold no more
+            float2 w[32];
+            cfor<0, 16>([&](auto j) {
+                constexpr int J = decltype(j)::value;
+                v[J] = sample(J);
+                w[J] = load2(bw, 8 * n0, 8 * STEP * J);
+            });
+            cfor<16, 32>([&](auto j) { v[decltype(j)::value] = sample(decltype(j)::value); });
+            __builtin_amdgcn_sched_barrier(0);
+            cfor<0, 32>([&](auto j) {
+                constexpr int J = decltype(j)::value;
+                v[J] = make_float2(v[J].x * w[J].x, v[J].y * w[J].y);
+                if constexpr (J < 16)
+                    w[J + 16] = load2(bw, 8 * n0, 8 * STEP * (J + 16));
+                if constexpr (J % 4 == 3)
+                    __builtin_amdgcn_sched_barrier(0);
+            });
+        } else {
+            cfor<0, 32>([&](auto j) { v[decltype(j)::value] = sample(decltype(j)::value); });
         }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            const uint32_t c = 2u * (e % CH), m = e / CH;
-            lds[c * PADR + pad(m)] = make_float2(xv[j].x * wv[j].x, xv[j].y * wv[j].y);
-            lds[(c + 1) * PADR + pad(m)] = make_float2(xv[j].z * wv[j].z, xv[j].w * wv[j].w);
-        }
-    } else if ((reinterpret_cast<uintptr_t>(a.sig + fs) & 7u) == 0 && inside) {
-        // the whole block lies inside the signal and its pairs are 8-byte
-        // aligned: every load is issued before the first one is used
-        float2 xv[16], wv[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            const uint32_t n = g0 + e % CB + (e / CB) * stride;
-            xv[j] = *reinterpret_cast<const float2*>(a.sig + fs + 2ull * n);
-            wv[j] = win2 ? win2[n] : make_float2(1.0f, 1.0f);
-        }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            lds[(e % CB) * PADR + pad(e / CB)] = make_float2(xv[j].x * wv[j].x, xv[j].y * wv[j].y);
-        }
+    };
+    if (fs + 2 * (uint64_t)(g0 + C + STRIDE * (R - 1)) <= a.L) {  // the workgroup's samples are all there
+        const auto bx = buffer(a.sig + fs, 8 * M);
+        window([&](uint32_t j) { return load2(bx, 8 * n0, 8 * STEP * j); });
     } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            const uint32_t c = e % CB, m = e / CB;
-            const uint32_t n = g0 + c + m * stride;
-            const uint64_t s0 = fs + 2ull * n;
-            const float2 w = win2 ? win2[n] : make_float2(1.0f, 1.0f);
-            float2 xv;
-            xv.x = s0 < a.L ? a.sig[s0] : 0.0f;
-            xv.y = s0 + 1 < a.L ? a.sig[s0 + 1] : 0.0f;
-            lds[c * PADR + pad(m)] = make_float2(xv.x * w.x, xv.y * w.y);
-        }
+        const float* x = a.sig + fs;
+        const uint64_t left = fs < a.L ? a.L - fs : 0;
+        window([&](uint32_t j) {
+            const uint32_t s = 2 * (n0 + STEP * j);
+            return make_float2(s < left ? x[s] : 0.0f, s + 1 < left ? x[s + 1] : 0.0f);
+        });
     }
-    __syncthreads();
 
-    const uint32_t col = tid / T, t = tid % T;
-    float2* z = lds + col * PADR;
-    float2 v[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-        v[j] = z[pad(t + j * T)];
+    Twist<32> none, tw;
+    twisted_dft<32, 0, 1, false>(v, none);
+    // twist of the second step's butterfly t: W_R^t
+    cfor<0, 5>([&](auto l) { tw.base[decltype(l)::value] = a.tw_r[t * (16u >> decltype(l)::value)]; });
+    float* const wr = lds + (32 * C + PAD) * t + c;
+    const float* const rd = lds + tid;
+    cfor<0, 32>([&](auto q) { wr[C * decltype(q)::value] = v[decltype(q)::value].x; });
     __syncthreads();
-    stockham<LOG_R, 0>(v, z, tws, t);
+    gather_step<C, 32, PAD, T, 1, 0>(v, rd);
+    __syncthreads();
+    cfor<0, 32>([&](auto q) { wr[C * decltype(q)::value] = v[decltype(q)::value].y; });
+    __syncthreads();
+    gather_step<C, 32, PAD, T, 1, 1>(v, rd);
+    twisted_dft<32, 0, 1, true>(v, tw);
 
-    // Y[g R + q]: each butterfly's R outputs are contiguous
-    const uint64_t obase = (P - a.frame0) * M + ((uint64_t)g0 << LOG_R);
-    if constexpr (OSTFT_MP_VEC4_ST) {
-        // two neighbouring outputs of a butterfly per 16-byte store (obase
-        // and e even)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t e = 2u * (tid + MP_THREADS * j);
-            const uint32_t c = e >> LOG_R, q = e & (R - 1);
-            const float2 v0 = lds[c * PADR + pad(q)], v1 = lds[c * PADR + pad(q + 1)];
-            *reinterpret_cast<float4*>(a.dst + obase + e) = make_float4(v0.x, v0.y, v1.x, v1.y);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t e = tid + MP_THREADS * j;
-            const uint32_t c = e >> LOG_R, q = e & (R - 1);
-            a.dst[obase + e] = lds[c * PADR + pad(q)];
-        }
-    }
+    // value i is row k = t + T i of column c
+    const auto bd = buffer(a.dst + (P - a.frame0) * M + (uint64_t)(g0 / MP_RUN) * (MP_RUN * R), 8 * MP_RUN * R);
+    cfor<0, 32>([&](auto i) {
+        constexpr int I = decltype(i)::value;
+        store2(bd, 8 * (t * MP_RUN + g0 % MP_RUN + c), 8 * T * MP_RUN * I, v[I]);
+    });
 }
 
 struct LastArgs {
-    const float2* src;        // first pass output
-    const float2* tw_r;       // W_R^j, j < R
-    const float2* tw_fine;    // W_M^j, j < 2^fine_bits
-    const float2* tw_coarse;  // W_M^(j << fine_bits)
-    const float2* tw_n;       // W_N^k, k < M
-    const float2* tw_2r;      // W_2R^q = W_N^(q Ns), q < R
+    const float2* src;   // first pass output
+    const float2* tw_r;  // W_R1^j, j < R1
+    const float2* tw_n;  // W_N^k, k < M
+    // W_M^(k 2^j), k < R0: the powers the twists take, side by side for the
+    // butterflies of a wave (gathered from W_N^k, they would fetch as many
+    // bytes again as the scratch values)
+    const float2* tw_k[9];
     float* out;
     uint64_t frame0, frames, out_limit;  // frames [frame0, frames); scratch row 0 = frame0
-    uint32_t fine_bits, log_m;
     int32_t combine, out_mode, dc;
 };
 
-template <int LOG_R>
-__global__ void __launch_bounds__(MP_THREADS) last_pass_kernel(const LastArgs a)
+// Last pass: C / 2 butterflies k and their mirrors R0 - k (0 and R0/2 are their
+// own) of one frame, R points each with twist W_M^k: a step of r1 = R/16 points
+// and one of 16.  Loads have the lanes along a butterfly's inputs, where the
+// first pass left them side by side; the exchange turns the lanes along the
+// butterflies, where the output positions k + R0 q are side by side.
+template <int LOG_M, int THREADS>
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+    last_pass_kernel(const LastArgs a)
 {
-    constexpr int R = 1 << LOG_R, CB2 = MP_ELEMS / R, CB = CB2 / 2, T = R / 16, PADR = R + R / 16 + OSTFT_MP_COL_PAD;
-    static_assert(CB2 * T == MP_THREADS && CB >= 1, "MP_THREADS threads per block");
-    __shared__ float2 lds[CB2 * PADR];
+    constexpr uint32_t M = 1u << LOG_M, N = 2 * M, Ns = MP_R0, R = M / Ns;
+    constexpr uint32_t ELEMS = Tile<THREADS>::ELEMS, C = ELEMS / R, CB = C / 2, T = R / 32;
+    constexpr uint32_t r1 = R / 16, NC = 32 / r1;  // first step: NC columns a thread,
+    constexpr uint32_t CSTEP = THREADS / 16;       // so far apart
+    constexpr uint32_t PAD = 4;                    // spreads the 16 rows r1 t of a wave over the banks
+    constexpr uint32_t BPF = Ns / C;               // workgroups per frame
+    __shared__ __align__(16) float lds[Tile<THREADS>::LDS];
+    static_assert(Tile<THREADS>::LDS >= ELEMS + PAD * 16 && Tile<THREADS>::LDS >= ELEMS + 2, "exchanges");
 
     const uint32_t tid = threadIdx.x;
-    const uint64_t M = 1ull << a.log_m;
-    const uint32_t Ns = (uint32_t)(M >> LOG_R);  // butterflies of the pass (= its stride)
-    const uint64_t bpf = M / MP_ELEMS;           // blocks per frame = Ns / CB2
-    const uint64_t blk = xcd_block(blockIdx.x, gridDim.x);
-    const uint64_t P = a.frame0 + blk / bpf;
-    if (P >= a.frames)
-        return;  // uniform over the block
-    const uint32_t b = (uint32_t)(blk % bpf);
-    PassTwiddles<LOG_R> tws;
-    load_pass_twiddles<LOG_R>(tws, a.tw_r, tid % T);
-
+    // each XCD on frames of its own: neighbouring blocks, whose output runs
+    // share cache lines, meet in one L2 (plain order: 309 against 280 us at 2^18,
+    // 334 against 271 at 2^20)
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint64_t P = a.frame0 + blk / BPF;
+    const uint32_t b = blk % BPF;
     // column c < CB: butterfly b CB + c; column CB + h: its mirror Ns - (b CB + h),
     // with Ns/2 in the place of Ns (= butterfly 0, already in column 0)
     auto butterfly = [&](uint32_t c) -> uint32_t {
-        if (c < (uint32_t)CB)
-            return b * CB + c;
-        const uint32_t h = c - CB;
-        return (b == 0 && h == 0) ? Ns / 2 : Ns - (b * CB + h);
+        const uint32_t k = b * CB + (c & (CB - 1));
+        return c < CB ? k : k == 0 ? Ns / 2 : Ns - k;
     };
-    // The thread's 16 values share one column: c = tid mod CB2 (butterfly g),
-    // rows m = m0 + T j.  Inter-pass twiddle W_M^{g m} (g m < M): from the
-    // two-level FP64 table at every fourth row, and by products with
-    // W_M^{g T} in between (at most three chained roundings).
-    const uint32_t fmask = (1u << a.fine_bits) - 1u;
-    auto twiddle = [&](uint32_t ex) {
-        return cmul(a.tw_fine[ex & fmask], a.tw_coarse[ex >> a.fine_bits]);
-    };
-    const float2* src = a.src + (P - a.frame0) * M;
-    const uint32_t cc = tid % CB2, m0 = tid / CB2;
-    const uint32_t gc = butterfly(cc);
-    float2 xs[16];  // the scratch values first: nothing below waits on them until the product
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-        xs[j] = src[gc + (uint64_t)(m0 + T * j) * Ns];
-    // the epilogue's W_N^g and W_2R^q, loaded with the rest
-    float2 wg = make_float2(1.0f, 0.0f), w2r[16];
-    if (a.combine) {
-        wg = a.tw_n[gc];
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            w2r[j] = a.tw_2r[m0 + T * j];
+    // inputs g = t + 16 j of butterfly k: scratch [j][k][t]; columns cg + CSTEP i
+    float2 v[32];
+    {
+        const uint32_t t = tid & 15u, cg = tid >> 4;
+        const auto bs = buffer(a.src + (P - a.frame0) * M, 8 * M);
+        cfor<0, NC>([&](auto i) {
+            const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
+            cfor<0, r1>([&](auto j) {
+                v[decltype(i)::value * r1 + decltype(j)::value] =
+                    load2(bs, 8 * (k * MP_RUN + t), 8 * Ns * MP_RUN * decltype(j)::value);
+            });
+        });
+        float* const wr = lds + (r1 * C + PAD) * t + cg;
+        cfor<0, NC>([&](auto i) {
+            // twist over j: W_M^(16 k)
+            constexpr int O = decltype(i)::value * r1;
+            const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
+            Twist<r1> tw;
+            cfor<0, ilog2(r1)>([&](auto l) {
+                tw.base[decltype(l)::value] = a.tw_k[4 + ilog2(r1) - 1 - decltype(l)::value][k];
+            });
+            twisted_dft<r1, O, 1, true>(v, tw);
+            cfor<0, r1>([&](auto q) { wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[O + decltype(q)::value].x; });
+        });
+        const float* const rd = lds + tid;
+        __syncthreads();
+        gather_step<C, r1, PAD, T, 2, 0>(v, rd);
+        __syncthreads();
+        cfor<0, NC>([&](auto i) {
+            cfor<0, r1>([&](auto q) {
+                wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[decltype(i)::value * r1 + decltype(q)::value].y;
+            });
+        });
+        __syncthreads();
+        gather_step<C, r1, PAD, T, 2, 1>(v, rd);
     }
-    const float2 step = twiddle(gc * T);
-    float2 anchor[4];
-#pragma unroll
-    for (int j = 0; j < 16; j += 4)
-        anchor[j / 4] = twiddle(gc * (m0 + T * j));
-    float2 tw = anchor[0];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const uint32_t m = m0 + T * j;
-        tw = (j % 4 == 0) ? anchor[j / 4] : cmul(tw, step);
-        lds[cc * PADR + pad(m)] = cmul(xs[j], tw);
-    }
-    __syncthreads();
+    const uint32_t c = tid % C, t = tid / C, k = butterfly(c);
+    const float2 wt = a.tw_n[k + Ns * t];
+    // second step, butterfly t + T u over 16 inputs: twist W_M^k W_R^(t + T u)
+    cfor<0, 2>([&](auto u) {
+        constexpr int UU = decltype(u)::value;
+        Twist<16> tu;
+        cfor<0, 4>([&](auto l) {
+            constexpr uint32_t J = 3 - decltype(l)::value;
+            tu.base[decltype(l)::value] = cmul(a.tw_k[J][k], a.tw_r[(t + T * UU) << J]);
+        });
+        twisted_dft<16, UU, 2, true>(v, tu);
+    });
+    // value i is row q = t + T i of column c: Z[k + Ns q]
+    const bool k0 = b == 0 && c == 0;
+    if (a.dc && k0 && t == 0)  // subtracting the mean only moves Z[0]
+        v[0] = make_float2(0.5f * (v[0].x - v[0].y), 0.5f * (v[0].y - v[0].x));
 
-    const uint32_t col = tid / T, t = tid % T;
-    float2* z = lds + col * PADR;
-    float2 v[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j)
-        v[j] = z[pad(t + j * T)];
+    // mirrors: Z[M - (k + Ns q)] is row R - 1 - q of the mirror column (row R - q
+    // of column 0 for butterfly 0, with Z[0] as its row R).  The upper rows go
+    // through LDS.
+    float2* const zu = reinterpret_cast<float2*>(lds);  // [row - R/2][column]
     __syncthreads();
-    stockham<LOG_R, 0>(v, z, tws, t);
-    // column c, row q now holds Z[k], k = butterfly(c) + q Ns
+    cfor<16, 32>([&](auto i) { zu[tid + T * C * (decltype(i)::value - 16)] = v[decltype(i)::value]; });
+    if (k0 && t == 0)
+        zu[ELEMS / 2] = v[0];
+    __syncthreads();
+    const uint32_t mc = b == 0 && (c & (CB - 1)) == 0 ? c : c ^ CB;
+    const float2* const zm = zu + (R / 2 - 1 + (k0 ? 1 : 0) - t) * C + mc;
 
-    // split: Z[M - k] is column mirror(c), row R - 1 - q (row (R - q) mod R
-    // for butterfly 0).  The thread's bins are k = g + q Ns, q = m0 + T j, of
-    // its column c = cc: W_N^k = W_N^g W_2R^q.
-    uint32_t mc;
-    if (gc == 0 || (gc == Ns / 2 && b == 0))
-        mc = cc;
-    else
-        mc = cc < (uint32_t)CB ? cc + CB : cc - CB;
-    // one straight-line body per output layout and stage choice
-    auto epilogue = [&](auto mode_c, auto comb_c) {
+    auto epilogue = [&](auto mode_c, auto comb_c, auto cut_c) {
         constexpr int MODE = decltype(mode_c)::value;
         constexpr bool COMB = decltype(comb_c)::value;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const uint32_t q = m0 + T * j;
-            const uint32_t mq = gc == 0 ? (R - q) & (R - 1) : R - 1 - q;
-            const uint32_t k = gc + q * Ns;
-            const float2 wk = COMB ? cmul(wg, w2r[j]) : wg;
-            const BinPair bp = finish_bin(lds[cc * PADR + pad(q)], lds[mc * PADR + pad(mq)], wk, COMB,
-                                          a.dc && k == 0);
-            write_bin(a.out, MODE, P, (uint32_t)M, k, bp, a.out_limit);
+        constexpr bool CUT = decltype(cut_c)::value;  // HALF_COMPLEX: the frame that out_limit cuts short
+        constexpr bool HALF = MODE == OUT_POWER || MODE == OUT_HALF_SPECTRUM;
+        constexpr bool CPLX = MODE == OUT_HALF_COMPLEX || MODE == OUT_HALF_SPECTRUM;
+        constexpr uint32_t B = CPLX ? 8 : 4;      // bytes of an output value
+        constexpr uint32_t W = HALF ? M + 1 : N;  // values of a frame
+        const uint64_t base = P * W;
+        const auto bo = buffer(reinterpret_cast<char*>(a.out) + B * base, B * W);
+        const uint64_t room = a.out_limit > base ? a.out_limit - base : 0;
+        auto put = [&](uint32_t lane, uint32_t pos, float2 x2, bool conj) {  // value at position lane + pos
+            if constexpr (MODE == OUT_COMPAT_POWER)
+                store1(bo, B * lane, B * pos, compat_power(x2));
+            else if constexpr (MODE == OUT_MAGNITUDE)
+                store1(bo, B * lane, B * pos, magnitude(x2));
+            else if constexpr (MODE == OUT_POWER)
+                store1(bo, B * lane, B * pos, power_of(x2));
+            else if (!CUT || lane + pos < room)
+                store2(bo, B * lane, B * pos, conj ? conj_value_of(x2) : value_of(x2));
+        };
+        // bin k + Ns q gives positions k + Ns q and M further on, and by the
+        // conjugate symmetry of a real frame's spectrum the mirrored two
+        const uint32_t lo = k + Ns * t, hi = Ns * T - lo;  // M - (lo + Ns T i) = hi + Ns T (31 - i)
+        cfor<0, 16>([&](auto i) {
+            constexpr uint32_t I = decltype(i)::value, O = Ns * T * I;
+            const BinPair bp = finish_pair<COMB>(v[I], *(zm - T * C * I), COMB ? cmul(wt, root<64, I>()) : wt);
+            const bool first = I == 0 && k0 && t == 0;  // bin 0 has no mirror below N
+            put(lo, O, bp.lo, false);
+            if constexpr (HALF) {
+                if (COMB || first)
+                    put(hi, M - Ns * T - O, bp.hi, !first);
+                else
+                    put(hi, M - Ns * T - O, bp.lo, true);
+            } else {
+                put(lo, M + O, bp.hi, false);
+                if (!first) {
+                    put(hi, M - Ns * T - O, COMB ? bp.hi : bp.lo, true);
+                    put(hi, N - Ns * T - O, COMB ? bp.lo : bp.hi, true);
+                }
+            }
+        });
+        if (k0 && t == 0) {  // bin M/2, its own mirror
+            const BinPair bp = finish_pair<COMB>(v[16], v[16], make_float2(0.0f, -1.0f));
+            put(0, M / 2, bp.lo, false);
+            if constexpr (!HALF)
+                put(0, M + M / 2, bp.hi, false);
         }
     };
-    auto by_stage = [&](auto mode_c) {
-        if (a.combine)
-            epilogue(mode_c, std::true_type{});
-        else
-            epilogue(mode_c, std::false_type{});
+    // one straight-line body per output layout and stage choice: the reference's
+    // odd-exponent result stops before the last stage, in its own layouts
+    constexpr bool VAR_COMBINE = LOG_M % 2 == 0;
+    using No = std::false_type;
+    using Yes = std::true_type;
+    auto by_stage = [&](auto mode_c, auto cut_c) {
+        if constexpr (VAR_COMBINE) {
+            if (!a.combine) {
+                epilogue(mode_c, No{}, cut_c);
+                return;
+            }
+        }
+        epilogue(mode_c, Yes{}, cut_c);
     };
     switch (a.out_mode) {
-    case OUT_COMPAT_POWER: by_stage(std::integral_constant<int, OUT_COMPAT_POWER>{}); break;
-    case OUT_MAGNITUDE: by_stage(std::integral_constant<int, OUT_MAGNITUDE>{}); break;
-    case OUT_HALF_COMPLEX: by_stage(std::integral_constant<int, OUT_HALF_COMPLEX>{}); break;
-    case OUT_POWER: by_stage(std::integral_constant<int, OUT_POWER>{}); break;
-    case OUT_HALF_SPECTRUM: by_stage(std::integral_constant<int, OUT_HALF_SPECTRUM>{}); break;
+    case OUT_COMPAT_POWER: by_stage(std::integral_constant<int, OUT_COMPAT_POWER>{}, No{}); break;
+    case OUT_MAGNITUDE: by_stage(std::integral_constant<int, OUT_MAGNITUDE>{}, No{}); break;
+    case OUT_HALF_COMPLEX:
+        if ((P + 1) * N <= a.out_limit)
+            by_stage(std::integral_constant<int, OUT_HALF_COMPLEX>{}, No{});
+        else
+            by_stage(std::integral_constant<int, OUT_HALF_COMPLEX>{}, Yes{});
+        break;
+    case OUT_POWER: epilogue(std::integral_constant<int, OUT_POWER>{}, Yes{}, No{}); break;
+    case OUT_HALF_SPECTRUM: epilogue(std::integral_constant<int, OUT_HALF_SPECTRUM>{}, Yes{}, No{}); break;
     default: break;
     }
 }
 
-int multipass_plan(int log_m, int* lr)
-{
-    // two passes: the last radix small, so that a block and its mirror block
-    // (CB = 4096 / R1 butterflies each) write long runs of consecutive bins
-    // (R1 = 2^6: 256-byte runs of the real layouts; 2^8 gave 64-byte runs and
-    // a 4-5% slower large-window step, 2^9 was 1.7x slower), the first radix
-    // at most 2^11 (its column segments are CB = 8192 / R0 values)
-    if (log_m < 16 || log_m > 19)
-        return 0;
-    lr[1] = 6;
-    if (log_m - lr[1] > 11)
-        lr[1] = log_m - 11;
-    lr[0] = log_m - lr[1];
-    return 2;
-}
+namespace {
 
-template <int LOG_R>
-static hipError_t launch_first(const PassArgs& p, hipStream_t s)
+// f(integral_constant<int, LOG_M>) for a runtime log_m in 16 .. 19
+template <typename F>
+hipError_t with_log_m(int log_m, F&& f)
 {
-    const uint64_t blocks = (p.frames - p.frame0) * ((1ull << p.log_m) / MP_ELEMS);
-    if (blocks > 0x7fffffffull)
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(first_pass_kernel<LOG_R>, dim3((uint32_t)blocks), dim3(MP_THREADS), 0, s, p);
-    return hipGetLastError();
-}
-
-template <int LOG_R>
-static hipError_t launch_last(const LastArgs& p, hipStream_t s)
-{
-    const uint64_t blocks = (p.frames - p.frame0) * ((1ull << p.log_m) / MP_ELEMS);
-    if (blocks > 0x7fffffffull)
-        return hipErrorInvalidValue;
-    hipLaunchKernelGGL(last_pass_kernel<LOG_R>, dim3((uint32_t)blocks), dim3(MP_THREADS), 0, s, p);
-    return hipGetLastError();
-}
-
-static hipError_t first_pass(int log_r, const PassArgs& p, hipStream_t s)
-{
-    switch (log_r) {
-    case 10: return launch_first<10>(p, s);
-    case 11: return launch_first<11>(p, s);
+    switch (log_m) {
+    case 16: return f(std::integral_constant<int, 16>{});
+    case 17: return f(std::integral_constant<int, 17>{});
+    case 18: return f(std::integral_constant<int, 18>{});
+    case 19: return f(std::integral_constant<int, 19>{});
     default: return hipErrorInvalidValue;
     }
 }
 
-static hipError_t last_pass(int log_r, const LastArgs& p, hipStream_t s)
+template <int LOG_M, int THREADS>
+hipError_t launch_tiles(const PassArgs& p, const LastArgs& la, hipStream_t s)
 {
-    switch (log_r) {
-    case 6: return launch_last<6>(p, s);
-    case 7: return launch_last<7>(p, s);
-    case 8: return launch_last<8>(p, s);
-    default: return hipErrorInvalidValue;
-    }
+    const uint64_t blocks = (p.frames - p.frame0) * ((1u << LOG_M) / Tile<THREADS>::ELEMS);
+    if (blocks > 0x7fffffffull)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL((first_pass_kernel<LOG_M, THREADS>), dim3((uint32_t)blocks), dim3(THREADS), 0, s, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL((last_pass_kernel<LOG_M, THREADS>), dim3((uint32_t)blocks), dim3(THREADS), 0, s, la);
+    return hipGetLastError();
 }
+
+// Requests of up to so many values take the workgroups of 256 threads.  Per
+// call, 512 against 256 threads (overlap 0, default layout): window 2^17, 1 frame
+// 22.7 / 18.3 us, 16 frames (1.0 M values) 27.2 / 21.5, 64 (4.2 M) 37.3 / 37.4, 128
+// 68.0 / 79.0; 2^20, 4 frames (2.1 M) 31.3 / 29.1, 8 (4.2 M) 39.8 / 42.2, 16 71.7 / 95.7.
+constexpr uint64_t SMALL_VALUES = (uint64_t)192 * 16384;
+
+hipError_t launch_passes(int log_m, const PassArgs& p, const LastArgs& la, hipStream_t s)
+{
+    return with_log_m(log_m, [&](auto lc) -> hipError_t {
+        constexpr int LOG_M = decltype(lc)::value;
+        if ((p.frames - p.frame0) << LOG_M <= SMALL_VALUES)
+            return launch_tiles<LOG_M, 256>(p, la, s);
+        return launch_tiles<LOG_M, 512>(p, la, s);
+    });
+}
+
+}  // namespace
+
+bool multipass_supported(int log_m) { return log_m >= 16 && log_m <= 19; }
 
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m)
 {
@@ -441,40 +482,41 @@ namespace {
 // `noalloc` a table that is not resident yet is an error instead of being
 // built.
 struct PassTables {
-    const float2 *fine, *coarse, *r0, *r1, *r2r1;
-    uint32_t fine_bits;
+    const float2 *r0, *r1, *k[9] = {};
 };
 
-int pass_tables(ostft_ctx* ctx, int log_m, const int* lr, bool noalloc, PassTables* t)
+int pass_tables(ostft_ctx* ctx, int log_m, bool noalloc, PassTables* t)
 {
     int rc = OSTFT_OK;
-    const int64_t M = (int64_t)1 << log_m;
-    t->fine_bits = (uint32_t)(log_m + 1) / 2;
-    if (!(t->fine = ctx_twiddles(ctx, M, (int64_t)1 << t->fine_bits, &rc, noalloc)))
-        return rc;
-    if (!(t->coarse = ctx_twiddles(ctx, M >> t->fine_bits, M >> t->fine_bits, &rc, noalloc)))
-        return rc;
-    if (!(t->r0 = ctx_twiddles(ctx, (int64_t)1 << lr[0], (int64_t)1 << lr[0], &rc, noalloc)))
-        return rc;
-    if (!(t->r1 = ctx_twiddles(ctx, (int64_t)1 << lr[1], (int64_t)1 << lr[1], &rc, noalloc)))
-        return rc;
-    if (!(t->r2r1 = ctx_twiddles(ctx, (int64_t)2 << lr[1], (int64_t)1 << lr[1], &rc, noalloc)))
-        return rc;
-    return OSTFT_OK;
+    const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
+    if ((t->r0 = ctx_twiddles(ctx, MP_R0, MP_R0, &rc, noalloc)))
+        t->r1 = ctx_twiddles(ctx, R1, R1, &rc, noalloc);
+    for (int j = 0; rc == OSTFT_OK && j < log_m - MP_LOG_R0; ++j)
+        t->k[j] = ctx_twiddles(ctx, (int64_t)1 << (log_m - j), MP_R0, &rc, noalloc);
+    return rc;
 }
 
-// The fewest chunks of at most `cap` frames, of equal size (a request of
-// 2^k + 1 frames gets no one-frame chunk at its end).
-uint64_t even_chunk(uint64_t frames, uint64_t cap)
+// Frames of the next chunk with `left` frames to go and room for `cap`.  A
+// chunk of 768 workgroups (96 MiB of scratch) is still in the 256 MB memory-side
+// cache when the last pass reads it; what is left over joins the last chunk or
+// makes one of at least half the size, so that no launch is nearly empty.
+// Scratch of 64 / 96 / 128 / 256 / 1024 MiB, 2^26 samples, 75%, default layout:
+// window 2^17 894 / 848 / 866 / 997 / 892 us, 2^20 990 / 961 / 1011 / 1178 / 1154.
+constexpr uint64_t CHUNK_VALUES = (uint64_t)768 * 16384;
+uint64_t chunk_frames(uint64_t left, uint64_t cap, int log_m)
 {
-    const uint64_t nchunks = (frames + cap - 1) / cap;
-    return nchunks ? (frames + nchunks - 1) / nchunks : 1;
+    const uint64_t want = CHUNK_VALUES >> log_m;
+    if (cap < want + want / 2) {  // a small budget: equal chunks
+        const uint64_t n = (left + cap - 1) / cap;
+        return n ? (left + n - 1) / n : 1;
+    }
+    return left <= want + want / 2 ? left : want;
 }
 
-// Both passes over the request's frames, `chunk` frames at a time through
-// `buf` (chunk * M complex values).
-int run_chunks(ostft_ctx* ctx, int log_m, const int* lr, const FusedArgs& a, const PassTables& t, float2* buf,
-               uint64_t chunk, hipStream_t s)
+// Both passes over the request's frames, a chunk at a time through `buf`
+// (`cap` frames).
+int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& t, float2* buf, uint64_t cap,
+               hipStream_t s)
 {
     PassArgs p;
     p.sig = a.in;
@@ -483,30 +525,22 @@ int run_chunks(ostft_ctx* ctx, int log_m, const int* lr, const FusedArgs& a, con
     p.win = a.win;
     p.dst = buf;
     p.tw_r = t.r0;
-    p.log_m = (uint32_t)log_m;
 
     LastArgs la;
     la.src = buf;
     la.tw_r = t.r1;
-    la.tw_fine = t.fine;
-    la.tw_coarse = t.coarse;
     la.tw_n = a.tw_n;
-    la.tw_2r = t.r2r1;
+    std::copy(std::begin(t.k), std::end(t.k), la.tw_k);
     la.out = a.out;
     la.out_limit = a.out_limit;
-    la.fine_bits = t.fine_bits;
-    la.log_m = (uint32_t)log_m;
     la.combine = a.combine;
     la.out_mode = a.out_mode;
     la.dc = a.dc;
 
-    for (uint64_t f0 = 0; f0 < a.frames; f0 += chunk) {
-        const uint64_t f1 = a.frames - f0 < chunk ? a.frames : f0 + chunk;
+    for (uint64_t f0 = 0; f0 < a.frames; f0 = p.frames) {
         p.frame0 = la.frame0 = f0;
-        p.frames = la.frames = f1;
-        hipError_t e = first_pass(lr[0], p, s);
-        if (e == hipSuccess)
-            e = last_pass(lr[1], la, s);
+        p.frames = la.frames = f0 + chunk_frames(a.frames - f0, cap, log_m);
+        const hipError_t e = launch_passes(log_m, p, la, s);
         if (e != hipSuccess)
             return ctx_hip_fail(ctx, e, "multi-pass launch");
     }
@@ -547,31 +581,25 @@ hipError_t multipass_static_scratch_init(int device)
 
 int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 {
-    int lr[4];
-    if (multipass_plan(log_m, lr) != 2)
+    if (!multipass_supported(log_m))
         return OSTFT_ERR_UNSUPPORTED;
     const uint64_t M = 1ull << log_m;
     // one call at a time queues launches on the shared scratch; the event
     // chain (acquire / handoff) orders their GPU work across streams
     std::lock_guard<std::mutex> lk(ctx_scratch_mutex(ctx));
     Scratch& sc = ctx_scratch(ctx);
-    // Frames go through both passes a chunk at a time, so the scratch
-    // allocation stays bounded (1 GiB by default) whatever the signal
-    // length.  Chunks small enough for their scratch to stay in the 256 MB
-    // memory-side cache between the passes measured slower (64 MiB: +15%,
-    // 128 MiB: +3% on windows 2^16..2^20 when all of them came this way): the passes are not bound by the
-    // round trip's HBM traffic, and every chunk adds two launch tails.
-    const uint64_t chunk = even_chunk(a.frames, multipass_chunk_frames(sc.budget, log_m));
-    hipError_t e = sc.ensure((a.frames < chunk ? a.frames : chunk) * M);
+    const uint64_t most = (CHUNK_VALUES + CHUNK_VALUES / 2) >> log_m;  // of any chunk
+    const uint64_t cap = std::min(std::min(multipass_chunk_frames(sc.budget, log_m), most), a.frames);
+    hipError_t e = sc.ensure(cap * M);
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass scratch allocation");
     e = sc.acquire(s);
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass scratch ordering");
     PassTables t;
-    int rc = pass_tables(ctx, log_m, lr, false, &t);
+    int rc = pass_tables(ctx, log_m, false, &t);
     if (rc == OSTFT_OK)
-        rc = run_chunks(ctx, log_m, lr, a, t, sc.a, chunk, s);
+        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, s);
     if (rc != OSTFT_OK)
         return rc;
     e = sc.handoff(s);
@@ -580,8 +608,7 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 
 int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs& a, hipStream_t s)
 {
-    int lr[4];
-    if (multipass_plan(log_m, lr) != 2)
+    if (!multipass_supported(log_m))
         return OSTFT_ERR_UNSUPPORTED;
     const uint64_t frame_bytes = sizeof(float2) << log_m;
     if (frame_bytes > STATIC_SCRATCH_BYTES)
@@ -597,10 +624,10 @@ int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs&
     if (!buf)
         return ctx_fail(ctx, OSTFT_ERR_HIP, "fixed scratch of this device was not set up at context creation");
     PassTables t;
-    const int rc = pass_tables(ctx, log_m, lr, true, &t);
+    const int rc = pass_tables(ctx, log_m, true, &t);
     if (rc != OSTFT_OK)
         return rc;
-    return run_chunks(ctx, log_m, lr, a, t, buf, even_chunk(a.frames, STATIC_SCRATCH_BYTES / frame_bytes), s);
+    return run_chunks(ctx, log_m, a, t, buf, STATIC_SCRATCH_BYTES / frame_bytes, s);
 }
 
 }  // namespace ostft

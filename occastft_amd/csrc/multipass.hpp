@@ -47,7 +47,6 @@ uint64_t multipass_static_scratch_bytes();
 // as many as fit `budget` bytes of scratch, at least one.
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m);
 
-// Radix split of 2^log_m into the two passes (returns 2; 0 outside 16..19).
-int multipass_plan(int log_m, int* log_radix /* [4] */);
+bool multipass_supported(int log_m);  // complex sizes 2^16 .. 2^19
 
 }  // namespace ostft
