@@ -211,6 +211,11 @@ typedef struct ostft_job {
  * `hip_stream`, no wait.  Outputs must not overlap. */
 int ostft_run_batch_device(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, void* hip_stream);
 
+/* Floats each request's layout writes (ostft_geometry.out_floats), 0 for a
+ * request whose geometry is refused: what a caller needs to size the outputs of
+ * a batch, in one call.  Reads full_size and params of each job only. */
+int ostft_batch_out_floats(const ostft_job* jobs, uint32_t njobs, uint64_t* out_floats);
+
 /* Batch launch form of window exponent `exp` (6..15): blocks_per_cu > 0
  * selects the persistent form with that many workgroups per CU (clamped to
  * the occupancy limit; it also sets workgroup shape 0, the only one the

@@ -56,6 +56,7 @@ EXPORTS = (
     "ostft_abi_version",
     "ostft_window_coefficients",
     "ostft_run_batch_device",
+    "ostft_batch_out_floats",
     "ostft_run_strided_device",
     "ostft_activate_geometry",
     "ostft_batch_config",
@@ -191,6 +192,8 @@ def lib() -> ctypes.CDLL:
     u64p = ctypes.POINTER(ctypes.c_uint64)
     L.ostft_run_batch_device.restype = ctypes.c_int
     L.ostft_run_batch_device.argtypes = [vp, ctypes.POINTER(Job), ctypes.c_uint32, vp]
+    L.ostft_batch_out_floats.restype = ctypes.c_int
+    L.ostft_batch_out_floats.argtypes = [ctypes.POINTER(Job), ctypes.c_uint32, u64p]
     L.ostft_run_strided_device.restype = ctypes.c_int
     L.ostft_run_strided_device.argtypes = [vp, ctypes.POINTER(Params), vp, ctypes.c_uint64, ctypes.c_uint64,
                                            ctypes.c_uint32, vp, ctypes.c_uint64, vp]

@@ -569,6 +569,17 @@ int ostft_get_geometry(const ostft_params* params, uint64_t full_size, ostft_geo
     return rc;
 }
 
+int ostft_batch_out_floats(const ostft_job* jobs, uint32_t njobs, uint64_t* out_floats)
+{
+    if ((!jobs || !out_floats) && njobs > 0)
+        return OSTFT_ERR_INVALID_ARG;
+    for (uint32_t i = 0; i < njobs; ++i) {
+        Plan plan;
+        out_floats[i] = make_plan(&jobs[i].params, jobs[i].full_size, &plan, nullptr) == OSTFT_OK ? plan.g.out_floats : 0;
+    }
+    return OSTFT_OK;
+}
+
 int ostft_create(int32_t device, ostft_ctx** out)
 {
     if (!out)

@@ -55,6 +55,36 @@ def geometry(params: N.Params, full_size: int) -> dict:
     return g.as_dict()
 
 
+def _out_floats(params: N.Params, full_size: int) -> int:
+    """geometry(...)["out_floats"] alone."""
+    g = N.Geometry()
+    rc = N.lib().ostft_get_geometry(ctypes.byref(params), full_size, ctypes.byref(g))
+    if rc != N.OK:
+        raise STFTError(rc)
+    return g.out_floats
+
+
+def _stream_handle(stream, device) -> int:
+    """hipStream_t of a torch stream, or of torch's current stream on `device`."""
+    import torch
+
+    if stream is not None:
+        return stream.cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # without making a Stream object
+    return raw(device.index) if raw is not None else torch.cuda.current_stream(device).cuda_stream
+
+
+def _trim(out, n: int):
+    """The first n floats of a flat tensor."""
+    return out if out.dim() == 1 and out.numel() == n else out[:n]
+
+
+# N.Job as numpy fills it, a column at a time
+_JOB = np.dtype([("in_ptr", "u8"), ("full_size", "u8"), ("out_ptr", "u8"), ("out_cap", "u8"),
+                 ("params", f"V{ctypes.sizeof(N.Params)}")])
+assert _JOB.itemsize == ctypes.sizeof(N.Job)
+
+
 class Runner:
     """One engine context on one HIP device.  It may be shared by several host
     threads: host-buffer calls run concurrently on the context's staging
@@ -122,17 +152,17 @@ class Runner:
 
         if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
             raise ValueError("x must be a contiguous float32 tensor on the GPU")
-        g = geometry(params, x.numel())
+        n = x.numel()
+        n_out = _out_floats(params, n)
         if out is None:
-            out = torch.empty(max(g["out_floats"], 1), dtype=torch.float32, device=x.device)
+            out = torch.empty(max(n_out, 1), dtype=torch.float32, device=x.device)
         if out.dtype != torch.float32 or not out.is_cuda or not out.is_contiguous():
             raise ValueError("out must be a contiguous float32 tensor on the GPU")
-        s = stream if stream is not None else torch.cuda.current_stream(x.device)
-        rc = N.lib().ostft_run_device(self._h, ctypes.byref(params), ctypes.c_void_p(x.data_ptr()), x.numel(),
-                                      ctypes.c_void_p(out.data_ptr()), out.numel(), ctypes.c_void_p(s.cuda_stream))
+        rc = N.lib().ostft_run_device(self._h, ctypes.byref(params), x.data_ptr(), n, out.data_ptr(), out.numel(),
+                                      _stream_handle(stream, x.device))
         if rc != N.OK:
             raise STFTError(rc, self.last_error)
-        return out[: g["out_floats"]]
+        return _trim(out, n_out)
 
     def run_strided_device(self, x, params: N.Params, out=None, stream=None):
         """STFT of every row of a (count, L) float32 CUDA tensor in one launch
@@ -164,29 +194,35 @@ class Runner:
         output tensors, each trimmed to its layout's length."""
         import torch
 
-        arr = (N.Job * max(len(jobs), 1))()
-        outs = []
-        dev = None
-        for i, (x, params, out) in enumerate(jobs):
-            if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
-                raise ValueError("inputs must be contiguous float32 tensors on the GPU")
-            dev = x.device
-            try:
-                n_out = geometry(params, x.numel())["out_floats"]
-            except STFTError:
-                n_out = 0  # the engine rejects the batch and names this job
-            if out is None:
-                out = torch.empty(max(n_out, 4), dtype=torch.float32, device=x.device)
-            arr[i].in_ptr = x.data_ptr()
-            arr[i].full_size = x.numel()
-            arr[i].out_ptr = out.data_ptr()
-            arr[i].out_cap = out.numel()
-            arr[i].params = params
-            outs.append(out[:n_out])
         if not jobs:
             return []
-        s = stream if stream is not None else torch.cuda.current_stream(dev)
-        rc = N.lib().ostft_run_batch_device(self._h, arr, len(jobs), ctypes.c_void_p(s.cuda_stream))
+        count = len(jobs)
+        ptrs, sizes, params = [], [], []
+        for x, p, _ in jobs:
+            if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
+                raise ValueError("inputs must be contiguous float32 tensors on the GPU")
+            ptrs.append(x.data_ptr())
+            sizes.append(x.numel())
+            params.append(bytes(p))
+        dev = x.device
+        table = np.zeros(count, dtype=_JOB)
+        table["in_ptr"] = ptrs
+        table["full_size"] = sizes
+        table["params"] = np.frombuffer(b"".join(params), dtype=_JOB["params"])
+        arr = (N.Job * count).from_buffer(table)
+        floats = (ctypes.c_uint64 * count)()
+        # 0 for a refused geometry: the engine rejects the batch below and names the job
+        N.lib().ostft_batch_out_floats(arr, count, floats)
+        outs, ptrs, caps = [], [], []
+        for (x, _, out), n_out in zip(jobs, floats):
+            if out is None:
+                out = torch.empty(max(n_out, 4), dtype=torch.float32, device=x.device)
+            outs.append(_trim(out, n_out))
+            ptrs.append(out.data_ptr())
+            caps.append(out.numel())
+        table["out_ptr"] = ptrs
+        table["out_cap"] = caps
+        rc = N.lib().ostft_run_batch_device(self._h, arr, count, _stream_handle(stream, dev))
         if rc != N.OK:
             raise STFTError(rc, self.last_error)
         return outs
