@@ -220,9 +220,9 @@ int ostft_batch_out_floats(const ostft_job* jobs, uint32_t njobs, uint64_t* out_
  * selects the persistent form with that many workgroups per CU (clamped to
  * the occupancy limit; it also sets workgroup shape 0, the only one the
  * persistent kernel is built for), < 0 the one-workgroup-per-tile form (the
- * default), 0 leaves it; use_graphs 0/1 turns replay of captured launch
- * sequences off/on (-1 leaves it; exp 0 sets only that); *current receives
- * the setting in force (0 for one workgroup per tile). */
+ * default), 0 leaves it (exp 0 too); use_graphs has no effect: launches are
+ * direct, which is faster than replaying captured ones for every mix of window
+ * sizes; *current receives the setting in force (0 for one workgroup per tile). */
 int ostft_batch_config(ostft_ctx* ctx, int32_t exp, int32_t blocks_per_cu, int32_t use_graphs,
                        int32_t* current);
 
@@ -291,7 +291,7 @@ typedef struct ostft_server_config {
     uint64_t arena_bytes;   /* device arena for admitted requests; 0: 1 GiB */
     uint32_t max_batch;     /* requests per batch; 0: 512 */
     uint32_t max_inflight;  /* batches on the GPU at once; 0: 3 */
-    int32_t use_graphs;     /* 1 (default when the config is NULL): replay captured launches */
+    int32_t use_graphs;     /* no effect (see ostft_batch_config) */
     int32_t autotune;       /* 1: autotune every batch window size (ostft_autotune_batch) at creation */
     const ostft_params* autotune_like; /* the requests to tune for (NULL: ostft_autotune_batch's default);
                                           read at creation only */

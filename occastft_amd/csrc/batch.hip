@@ -5,11 +5,14 @@
 // form, the workgroup shape (G) and the radix plan of each class are measured
 // by the autotuner.
 //
-// The descriptor block (per-class headers, the requests' FusedArgs, the
-// tile -> request table) is built on the host in pinned memory and uploaded
-// with one copy before the launches.  The launches themselves only name the
-// block, so for a given set of classes they are the same every time: they are
-// captured once into a HIP graph and replayed.
+// The requests' records are built on the host in pinned memory; a small kernel
+// ahead of the launches copies them to the descriptor block and writes the tile
+// -> request table there.  (With an upload of records and table by a copy in
+// the stream, the GPU stood idle 35-50 us between two batches: 9 before the
+// copy, 9 for 200 KB, 17-33 after it.)  The launches are made one by one: replaying
+// them from a captured graph with a node for each of the ten window sizes took
+// longer for every mix, 58 against 35 us a batch of 24 requests of three sizes, 280
+// against 274 us one of 256 requests of ten.
 //
 // Requests of windows >= 2^16 (one launch, or the two-pass path) and requests of the matrix-core
 // form run after the tile-queue launches, one request at a time, on the same
@@ -36,13 +39,23 @@ constexpr size_t ALIGN = 256;
 
 size_t align_up(size_t x) { return (x + ALIGN - 1) & ~(ALIGN - 1); }
 
-// One descriptor block: device copy, pinned host mirror, and the event after
-// the last launch that reads it (the mirror and the block are reused only
-// after it).
+// A request as the host writes it.
+struct BatchUpload {
+    BatchJob job;
+    uint64_t tiles_at;  // its first entry of the block's tile table
+    uint32_t ntiles;
+    uint32_t index;     // its place in its class
+};
+static_assert(sizeof(BatchJob) % 8 == 0 && sizeof(BatchUpload) % 8 == 0, "copied by 8-byte words");
+
+// One descriptor block (claim counters, BatchJob records, tile table), the
+// pinned records it is filled from, and the event after the last launch that
+// reads it (both are reused only after it).
 struct Slot {
     char* d = nullptr;
-    char* h = nullptr;
-    size_t cap = 0;
+    size_t d_cap = 0;
+    BatchUpload* h = nullptr;
+    size_t h_cap = 0;  // records
     hipEvent_t done = nullptr;
     bool used = false;
 };
@@ -53,7 +66,6 @@ struct BatchState {
     Slot slot[2];
     int next = 0;
     int cu_count = 0;
-    int use_graphs = 1;
     int persistent[NCLS] = {};  // 1: persistent grid claiming tiles; 0: one workgroup per tile
     int per_cu[NCLS] = {};      // persistent workgroups per CU; 0: the occupancy limit
     int shape[NCLS] = {};       // workgroup shape (engine variant / 4); persistent needs 0
@@ -61,35 +73,11 @@ struct BatchState {
     int variant[NCLS] = {};     // engine variant of each class in the current batch
     BatchClassInfo info[NCLS][FUSED_VARIANTS] = {};
     bool info_ok[NCLS][FUSED_VARIANTS] = {};
-    // per slot: the launches of every class, captured once; a batch sets
-    // each class node's grid (its persistent grid, or one workgroup when the
-    // class has no tiles) and replays it
-    hipGraph_t graph[2] = {};
-    hipGraphExec_t exec[2] = {};
-    hipGraphNode_t node[2][NCLS] = {};
-    uint32_t node_grid[2][NCLS] = {};
-    int node_persistent[2][NCLS] = {};
-    int node_variant[2][NCLS] = {};
-    hipStream_t capture = nullptr;
 
     BatchState()
     {
         for (int& p : plan_override)
             p = -1;
-    }
-    void drop_graph(int i)
-    {
-        if (exec[i])
-            (void)hipGraphExecDestroy(exec[i]);
-        if (graph[i])
-            (void)hipGraphDestroy(graph[i]);
-        exec[i] = nullptr;
-        graph[i] = nullptr;
-    }
-    void drop_graphs()
-    {
-        for (int i = 0; i < 2; ++i)
-            drop_graph(i);
     }
 };
 
@@ -102,13 +90,9 @@ int state(ostft_ctx* ctx, BatchState** out)
         BatchState* s = new BatchState();
         hipDeviceProp_t prop;
         hipError_t e = hipGetDeviceProperties(&prop, ctx_device(ctx));
-        if (e == hipSuccess)
-            e = hipStreamCreateWithFlags(&s->capture, hipStreamNonBlocking);
         for (int i = 0; e == hipSuccess && i < 2; ++i)
             e = hipEventCreateWithFlags(&s->slot[i].done, hipEventDisableTiming);
         if (e != hipSuccess) {
-            if (s->capture)
-                (void)hipStreamDestroy(s->capture);
             for (auto& sl : s->slot)
                 if (sl.done)
                     (void)hipEventDestroy(sl.done);
@@ -153,140 +137,53 @@ uint32_t class_grid(const BatchState* st, int c, uint64_t ntiles)
     return (uint32_t)pc * (uint32_t)st->cu_count;
 }
 
-hipError_t launch_classes(BatchState* st, uint32_t mask, void* base, hipStream_t s, const uint64_t* ntiles,
-                          bool one_block = false)
+// Workgroup (j, y) of `parts` per request: part y of request j's entries of the
+// tile table, and its record.
+constexpr int FILL_THREADS = 256;
+__global__ void __launch_bounds__(FILL_THREADS)
+    batch_fill_kernel(const BatchUpload* __restrict__ up, BatchJob* __restrict__ jobs, uint32_t* __restrict__ tiles,
+                      uint32_t* __restrict__ counters)
 {
-    for (int c = 0; c < NCLS; ++c) {
-        if (!(mask >> c & 1u))
-            continue;
-        BatchClassArgs a;
-        a.base = base;
-        a.header_off = (uint64_t)c * sizeof(BatchClassHeader);
-        const uint32_t grid = one_block ? 1u : class_grid(st, c, ntiles[c]);
-        const hipError_t e = launch_batch(c + LOG_M_MIN, st->variant[c], a, grid, st->persistent[c] != 0, s);
-        if (e != hipSuccess)
-            return e;
-    }
-    return hipSuccess;
+    const uint32_t j = blockIdx.x, tid = threadIdx.x;
+    const BatchUpload* u = up + j;
+    const uint64_t at = u->tiles_at;
+    const uint32_t n = u->ntiles, index = u->index;
+    if (blockIdx.y == 0 && tid < sizeof(BatchJob) / 8)
+        reinterpret_cast<uint64_t*>(jobs + j)[tid] = reinterpret_cast<const uint64_t*>(&u->job)[tid];
+    if (j == 0 && blockIdx.y == 0 && tid < NCLS)
+        counters[tid] = 0;
+    for (uint64_t i = blockIdx.y * FILL_THREADS + tid; i < n; i += (uint64_t)gridDim.y * FILL_THREADS)
+        tiles[at + i] = index;
 }
 
-// Captures the launches of every class for slot `si` (grids of one
-// workgroup; set per batch) and finds each class's kernel node.
-hipError_t capture_slot(BatchState* st, int si)
+hipError_t ensure_slot(Slot& sl, size_t d_bytes, size_t records)
 {
-    const uint32_t all = (1u << NCLS) - 1u;
-    hipGraph_t g = nullptr;
-    hipError_t e = hipStreamBeginCapture(st->capture, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess)
-        return e;
-    const hipError_t le = launch_classes(st, all, st->slot[si].d, st->capture, nullptr, true);
-    e = hipStreamEndCapture(st->capture, &g);
-    if (le != hipSuccess || e != hipSuccess) {
-        if (g)
-            (void)hipGraphDestroy(g);
-        return le != hipSuccess ? le : e;
-    }
-    // the captured graph is the chain class 0 -> class NCLS-1
-    for (int c = 0; c < NCLS; ++c)
-        st->node[si][c] = nullptr;
-    size_t n = 0;
-    e = hipGraphGetNodes(g, nullptr, &n);
-    std::vector<hipGraphNode_t> nodes(n);
-    if (e == hipSuccess && n == (size_t)NCLS)
-        e = hipGraphGetNodes(g, nodes.data(), &n);
-    else if (e == hipSuccess)
-        e = hipErrorInvalidValue;
-    for (size_t i = 0; e == hipSuccess && i < n; ++i) {
-        hipKernelNodeParams kp;
-        e = hipGraphKernelNodeGetParams(nodes[i], &kp);
-        if (e != hipSuccess)
-            break;
-        int c = -1;
-        for (int k = 0; k < NCLS; ++k)
-            if (kp.func == batch_kernel_fn(k + LOG_M_MIN, st->variant[k], st->persistent[k] != 0))
-                c = k;
-        if (c < 0 || st->node[si][c]) {
-            e = hipErrorInvalidValue;
-            break;
-        }
-        st->node[si][c] = nodes[i];
-        st->node_grid[si][c] = 1;
-        st->node_persistent[si][c] = st->persistent[c];
-        st->node_variant[si][c] = st->variant[c];
-    }
-    hipGraphExec_t ex = nullptr;
-    if (e == hipSuccess)
-        e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(g);
-        return e;
-    }
-    st->graph[si] = g;
-    st->exec[si] = ex;
-    return hipSuccess;
-}
-
-// Replays slot `si`'s launches with the grids this batch needs.
-hipError_t replay_slot(BatchState* st, int si, uint32_t mask, const uint64_t* ntiles, hipStream_t s)
-{
-    for (int c = 0; st->exec[si] && c < NCLS; ++c)
-        if (st->node_persistent[si][c] != st->persistent[c] || st->node_variant[si][c] != st->variant[c]) {
-            // a class changed form or variant: its node names another kernel
-            (void)hipGraphExecDestroy(st->exec[si]);
-            (void)hipGraphDestroy(st->graph[si]);
-            st->exec[si] = nullptr;
-            st->graph[si] = nullptr;
-        }
-    if (!st->exec[si]) {
-        const hipError_t e = capture_slot(st, si);
-        if (e != hipSuccess)
-            return e;
-    }
-    for (int c = 0; c < NCLS; ++c) {
-        const uint32_t want = (mask >> c & 1u) ? class_grid(st, c, ntiles[c]) : 1u;
-        if (want == st->node_grid[si][c])
-            continue;
-        hipKernelNodeParams kp;
-        hipError_t e = hipGraphKernelNodeGetParams(st->node[si][c], &kp);
-        if (e != hipSuccess)
-            return e;
-        kp.gridDim = dim3(want);
-        e = hipGraphExecKernelNodeSetParams(st->exec[si], st->node[si][c], &kp);
-        if (e != hipSuccess)
-            return e;
-        st->node_grid[si][c] = want;
-    }
-    return hipGraphLaunch(st->exec[si], s);
-}
-
-hipError_t ensure_slot(BatchState* st, int si, size_t bytes)
-{
-    Slot& sl = st->slot[si];
-    if (sl.cap >= bytes)
-        return hipSuccess;
-    // this slot's captured launches name the old block: drop them (nothing
-    // in flight reads it: the caller waited on the slot's event); the other
-    // slot's graph names its own block and may still be running
-    st->drop_graph(si);
-    if (sl.d)
-        (void)hipFree(sl.d);
-    if (sl.h)
-        (void)hipHostFree(sl.h);
-    sl.d = nullptr;
-    sl.h = nullptr;
-    sl.cap = 0;
-    const size_t cap = std::max<size_t>(align_up(bytes + bytes / 2), 64 * 1024);
-    hipError_t e = hipMalloc(&sl.d, cap);
-    if (e == hipSuccess)
-        e = hipHostMalloc(&sl.h, cap, hipHostMallocDefault);
-    if (e != hipSuccess) {
+    if (sl.d_cap < d_bytes) {
         if (sl.d)
             (void)hipFree(sl.d);
         sl.d = nullptr;
-        sl.h = nullptr;
-        return e;
+        sl.d_cap = 0;
+        const size_t cap = std::max<size_t>(align_up(d_bytes + d_bytes / 2), 64 * 1024);
+        const hipError_t e = hipMalloc(&sl.d, cap);
+        if (e != hipSuccess) {
+            sl.d = nullptr;
+            return e;
+        }
+        sl.d_cap = cap;
     }
-    sl.cap = cap;
+    if (sl.h_cap < records) {
+        if (sl.h)
+            (void)hipHostFree(sl.h);
+        sl.h = nullptr;
+        sl.h_cap = 0;
+        const size_t cap = std::max<size_t>(records + records / 2, 256);
+        const hipError_t e = hipHostMalloc(&sl.h, cap * sizeof(BatchUpload), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            sl.h = nullptr;
+            return e;
+        }
+        sl.h_cap = cap;
+    }
     return hipSuccess;
 }
 
@@ -356,17 +253,20 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         if (ntiles[c] >= 0x7fffffffull - 2ull * (uint64_t)st->cu_count * 64u)  // grid limit; claims overrun by <= 2/workgroup
             return ctx_fail(ctx, OSTFT_ERR_TOO_LARGE, "more than 2^31 tiles of one window size in a batch");
     if (mask) {
-        // 3. descriptor block layout
-        size_t off = align_up(sizeof(BatchClassHeader) * NCLS);
-        size_t jobs_off[NCLS] = {}, tiles_off[NCLS] = {};
+        // 3. descriptor block layout: claim counters, requests class by class,
+        //    tile tables class by class
+        size_t nreq = 0;
+        uint64_t total = 0, most = 0;
+        size_t first_job[NCLS] = {};
+        uint64_t first_tile[NCLS] = {};
         for (int c = 0; c < NCLS; ++c) {
-            if (!(mask >> c & 1u))
-                continue;
-            jobs_off[c] = off;
-            off = align_up(off + sizeof(BatchJob) * members[c].size());
-            tiles_off[c] = off;
-            off = align_up(off + sizeof(uint32_t) * ntiles[c]);
+            first_job[c] = nreq;
+            first_tile[c] = total;
+            nreq += members[c].size();
+            total += ntiles[c];
         }
+        const size_t jobs_off = align_up(sizeof(uint32_t) * NCLS);
+        const size_t tiles_off = align_up(jobs_off + sizeof(BatchJob) * nreq);
         const int si = st->next;
         st->next ^= 1;
         Slot& sl = st->slot[si];
@@ -375,42 +275,41 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
             if (e != hipSuccess)
                 return ctx_hip_fail(ctx, e, "batch slot wait");
         }
-        hipError_t e = ensure_slot(st, si, off);
+        hipError_t e = ensure_slot(sl, tiles_off + sizeof(uint32_t) * total, nreq);
         if (e != hipSuccess)
             return ctx_hip_fail(ctx, e, "batch descriptor block");
-        // 4. fill the pinned mirror
-        BatchClassHeader* hdr = reinterpret_cast<BatchClassHeader*>(sl.h);
-        std::memset(hdr, 0, sizeof(BatchClassHeader) * NCLS);
+        // 4. the requests' records
         for (int c = 0; c < NCLS; ++c) {
-            if (!(mask >> c & 1u))
-                continue;
-            hdr[c].jobs_off = jobs_off[c];
-            hdr[c].tiles_off = tiles_off[c];
-            hdr[c].ntiles = (uint32_t)ntiles[c];
-            hdr[c].counter = 0;
-            BatchJob* bj = reinterpret_cast<BatchJob*>(sl.h + jobs_off[c]);
-            uint32_t* tj = reinterpret_cast<uint32_t*>(sl.h + tiles_off[c]);
             uint64_t t = 0;
             for (size_t k = 0; k < members[c].size(); ++k) {
-                const FusedArgs& a = args[members[c][k]];
-                bj[k].a = a;
-                bj[k].tile_begin = t;
-                const uint64_t nt = (a.frames + a.tile_frames - 1) / a.tile_frames;
-                std::fill(tj + t, tj + t + nt, (uint32_t)k);
+                BatchUpload& u = sl.h[first_job[c] + k];
+                u.job.a = args[members[c][k]];
+                u.job.tile_begin = t;
+                const uint64_t nt = (u.job.a.frames + u.job.a.tile_frames - 1) / u.job.a.tile_frames;
+                u.tiles_at = first_tile[c] + t;
+                u.ntiles = (uint32_t)nt;
+                u.index = (uint32_t)k;
                 t += nt;
+                most = std::max(most, nt);
             }
         }
-        // 5. upload, then the launches (replayed graph or direct)
-        e = hipMemcpyAsync(sl.d, sl.h, off, hipMemcpyHostToDevice, s);
-        if (e != hipSuccess)
-            return ctx_hip_fail(ctx, e, "batch descriptor upload");
-        // the captured sequence holds a node per window size (an absent size
-        // still costs one exiting workgroup, ~3.5 us): replay it when at least
-        // three sizes are present, launch directly otherwise
-        if (st->use_graphs && __builtin_popcount(mask) >= 3) {
-            e = replay_slot(st, si, mask, ntiles, s);
-        } else {
-            e = launch_classes(st, mask, sl.d, s, ntiles);
+        // 5. the descriptor block, then the launches
+        uint32_t* const counters = reinterpret_cast<uint32_t*>(sl.d);
+        BatchJob* const bj = reinterpret_cast<BatchJob*>(sl.d + jobs_off);
+        uint32_t* const tj = reinterpret_cast<uint32_t*>(sl.d + tiles_off);
+        const uint32_t parts = (uint32_t)std::min<uint64_t>(1 + most / (16 * FILL_THREADS), 256);
+        hipLaunchKernelGGL(batch_fill_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj, tj,
+                           counters);
+        e = hipGetLastError();
+        for (int c = 0; e == hipSuccess && c < NCLS; ++c) {
+            if (!(mask >> c & 1u))
+                continue;
+            BatchClassArgs a;
+            a.jobs = bj + first_job[c];
+            a.tile_job = tj + first_tile[c];
+            a.counter = counters + c;
+            a.ntiles = (uint32_t)ntiles[c];
+            e = launch_batch(c + LOG_M_MIN, st->variant[c], a, class_grid(st, c, ntiles[c]), st->persistent[c] != 0, s);
         }
         if (e == hipSuccess)
             e = hipEventRecord(sl.done, s);
@@ -452,21 +351,18 @@ int class_of(ostft_ctx* ctx, int exp, int* c)
 
 }  // namespace
 
-int batch_config(ostft_ctx* ctx, int exp, int blocks_per_cu, int use_graphs, int* current)
+int batch_config(ostft_ctx* ctx, int exp, int blocks_per_cu, int* current)
 {
     BatchState* st = nullptr;
     int rc = state(ctx, &st);
     if (rc != OSTFT_OK)
         return rc;
-    if (use_graphs >= 0)
-        st->use_graphs = use_graphs ? 1 : 0;
     if (exp == 0)
         return OSTFT_OK;
     int c = 0;
     rc = class_of(ctx, exp, &c);
     if (rc != OSTFT_OK)
         return rc;
-    // captured launches take a new setting at their next replay
     if (blocks_per_cu > 0) {
         const int v = ctx_radix_plan(ctx, c + LOG_M_MIN);  // shape 0
         rc = class_info(ctx, st, c, v);
@@ -626,9 +522,7 @@ int autotune_batch(ostft_ctx* ctx, int exp, uint64_t samples, const ostft_params
             j.in = din + reinterpret_cast<uint64_t>(j.in);
             j.out = dout + reinterpret_cast<uint64_t>(j.out);
         }
-        const int saved_graphs = st->use_graphs, saved_pc = st->per_cu[c], saved_ps = st->persistent[c],
-                  saved_shape = st->shape[c];
-        st->use_graphs = 0;
+        const int saved_pc = st->per_cu[c], saved_ps = st->persistent[c], saved_shape = st->shape[c];
         // the GPU time of one batch under candidate (variant, per CU): min
         // over `rounds` - 1 timed rounds after a warming one
         auto timed = [&](const std::pair<int, int>& cd, int rounds) {
@@ -687,12 +581,10 @@ int autotune_batch(ostft_ctx* ctx, int exp, uint64_t samples, const ostft_params
             }
         }
         st->plan_override[c] = -1;
-        st->use_graphs = saved_graphs;
         st->per_cu[c] = saved_pc;
         st->persistent[c] = saved_ps;
         st->shape[c] = saved_shape;
         if (rc == OSTFT_OK && e == hipSuccess) {
-            // captured launches take it at their next replay
             st->shape[c] = best.first >> 2;
             st->persistent[c] = best.second > 0;
             st->per_cu[c] = best.second;
@@ -739,9 +631,6 @@ void batch_release(ostft_ctx* ctx)
         if (sl.done)
             (void)hipEventDestroy(sl.done);
     }
-    b->drop_graphs();
-    if (b->capture)
-        (void)hipStreamDestroy(b->capture);
     delete b;
     b = nullptr;
 }

@@ -61,7 +61,7 @@ struct ostft_ctx {
     std::mutex scratch_mu;
     ostft::Scratch scratch;
     std::mutex batch_mu;
-    ostft::BatchState* batch = nullptr;  // batch descriptors, graphs, plans (batch.hip)
+    ostft::BatchState* batch = nullptr;  // batch descriptors, plans (batch.hip)
     std::mutex err_mu;
     std::unordered_map<std::thread::id, std::string> errors;  // last error per calling thread
     // radix plan of the single-kernel engine per complex size 2^log_m, read
@@ -773,7 +773,8 @@ int ostft_batch_config(ostft_ctx* ctx, int32_t exp, int32_t blocks_per_cu, int32
     if (!dg.ok)
         return fail(ctx, OSTFT_ERR_NO_DEVICE, "hipSetDevice failed");
     std::lock_guard<std::mutex> lk(ctx->batch_mu);
-    return ostft::batch_config(ctx, exp, blocks_per_cu, use_graphs, current);
+    (void)use_graphs;  // launches are direct either way
+    return ostft::batch_config(ctx, exp, blocks_per_cu, current);
 }
 
 int ostft_engine_variant(ostft_ctx* ctx, int32_t exp, int32_t shape, int32_t plan, int32_t* cur_shape,

@@ -80,23 +80,18 @@ hipError_t launch_fused(int log_m, int xf, const FusedArgs& a, uint32_t count, h
 bool wide_supported(int log_m);
 hipError_t launch_wide(const FusedArgs& a, uint32_t count, hipStream_t s);
 
-// ---- batches: many requests of one window size in one persistent launch ----
-// A batch descriptor block lives in device memory (uploaded by the host before
-// the launch); the kernel arguments only name where, so one captured launch
-// sequence serves every batch.
+// ---- batches: many requests of one window size in one launch ----
+// A batch descriptor block lives in device memory, filled on the stream before
+// the launches (batch.hip).
 struct BatchJob {
     FusedArgs a;
     uint64_t tile_begin;  // first tile of this request in its class
 };
-struct BatchClassHeader {
-    uint64_t jobs_off;    // byte offset of BatchJob[njobs] from the block base
-    uint64_t tiles_off;   // byte offset of uint32 tile_job[ntiles]
-    uint32_t ntiles;      // tiles of G frames in the class (0: the launch exits at once)
-    uint32_t counter;     // next unclaimed tile; uploaded as 0
-};
 struct BatchClassArgs {
-    void* base;           // descriptor block
-    uint64_t header_off;  // byte offset of this class's BatchClassHeader
+    const BatchJob* jobs;      // the class's requests
+    const uint32_t* tile_job;  // request of each tile
+    uint32_t* counter;         // next unclaimed tile, 0 before the launch (persistent form)
+    uint32_t ntiles;           // tiles of G frames in the class
 };
 struct BatchClassInfo {
     int frames_per_tile;    // G
@@ -108,8 +103,6 @@ struct BatchClassInfo {
 hipError_t launch_batch(int log_m, int variant, const BatchClassArgs& b, uint32_t grid, bool persistent,
                         hipStream_t s);
 hipError_t batch_class_info(int log_m, int variant, BatchClassInfo* info);
-// the kernel's host handle (graph nodes name it)
-const void* batch_kernel_fn(int log_m, int variant, bool persistent);
 
 // FP64 table generators (run once per table).
 // tw[j] = exp(-2 pi i j / m) for j < count (count <= m)

@@ -920,19 +920,13 @@ __global__ void __launch_bounds__((Cfg<LOG_M, PLAN>::WG)) __attribute__((amdgpu_
 // (ostft_autotune_batch).
 template <int LOG_M, int V>
 __global__ void __launch_bounds__((Cfg<LOG_M, V>::WG)) __attribute__((amdgpu_waves_per_eu(4)))
-    stft_batch_dispatch_kernel(const char* __restrict__ blk, const uint32_t header_off)
+    stft_batch_dispatch_kernel(const BatchJob* __restrict__ jobs, const uint32_t* __restrict__ tile_job)
 {
     using C = Cfg<LOG_M, V>;
     __shared__ float2 lds[C::G * C::PADM];
     __shared__ float2 red[C::WG / 64];
-    const BatchClassHeader* h = reinterpret_cast<const BatchClassHeader*>(blk + header_off);
-    const uint32_t ntiles = h->ntiles;
-    // the grid is ntiles (or 1 for an empty class): a permutation of the tiles
-    const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);
-    if (tile >= ntiles)
-        return;
-    const BatchJob* jobs = reinterpret_cast<const BatchJob*>(blk + h->jobs_off);
-    const uint32_t j = reinterpret_cast<const uint32_t*>(blk + h->tiles_off)[tile];
+    const uint32_t tile = xcd_block(blockIdx.x, gridDim.x);  // a permutation of the tiles
+    const uint32_t j = tile_job[tile];
     const FusedArgs a = from_global(*reinterpret_cast<const FusedArgsGlobal*>(&jobs[j].a));
     fused_frames<LOG_M, V>(a, (uint64_t)(tile - jobs[j].tile_begin) * (uint32_t)a.tile_frames, lds, red,
                            threadIdx.x);
@@ -941,18 +935,15 @@ __global__ void __launch_bounds__((Cfg<LOG_M, V>::WG)) __attribute__((amdgpu_wav
 template <int LOG_M, int PLAN>
 __global__ void __launch_bounds__((Cfg<LOG_M, PLAN>::WG))
     __attribute__((amdgpu_waves_per_eu(BatchWaves<LOG_M>::value)))
-    stft_batch_kernel(const char* __restrict__ blk, uint32_t* __restrict__ counter, const uint32_t header_off)
+    stft_batch_kernel(const BatchJob* __restrict__ jobs, const uint32_t* __restrict__ tile_job,
+                      uint32_t* __restrict__ counter, const uint32_t ntiles)
 {
-    // `blk` is read-only here (the counter is reached only through `counter`),
-    // which lets the compiler read the descriptors with scalar loads
+    // the descriptors are read-only here (the counter is apart), which lets the
+    // compiler read them with scalar loads
     using C = Cfg<LOG_M, PLAN>;
     __shared__ float2 lds[C::G * C::PADM];
     __shared__ float2 red[C::WG / 64];
     __shared__ uint32_t claim;
-    const BatchClassHeader* h = reinterpret_cast<const BatchClassHeader*>(blk + header_off);
-    const uint32_t ntiles = h->ntiles;
-    const BatchJob* jobs = reinterpret_cast<const BatchJob*>(blk + h->jobs_off);
-    const uint32_t* tile_job = reinterpret_cast<const uint32_t*>(blk + h->tiles_off);
     if (threadIdx.x == 0)
         claim = atomicAdd(counter, 1u);
     __syncthreads();
@@ -1064,22 +1055,21 @@ static hipError_t launch_batch_t(int v, const BatchClassArgs& b, uint32_t grid, 
 {
     if (grid == 0)
         return hipErrorInvalidValue;
-    char* blk = static_cast<char*>(b.base);
     return with_variant<LOG_M>(v, [&](auto vc) -> hipError_t {
         constexpr int V = decltype(vc)::value;
         using C = Cfg<LOG_M, V>;
         if (persistent) {
             if constexpr (C::SHAPE == 0) {
-                uint32_t* counter =
-                    reinterpret_cast<uint32_t*>(blk + b.header_off + offsetof(BatchClassHeader, counter));
-                hipLaunchKernelGGL((stft_batch_kernel<LOG_M, C::PLAN>), dim3(grid), dim3(C::WG), 0, s,
-                                   static_cast<const char*>(blk), counter, (uint32_t)b.header_off);
+                hipLaunchKernelGGL((stft_batch_kernel<LOG_M, C::PLAN>), dim3(grid), dim3(C::WG), 0, s, b.jobs,
+                                   b.tile_job, b.counter, b.ntiles);
             } else {
                 return hipErrorInvalidValue;  // the persistent form has workgroup shape 0 only
             }
         } else {
-            hipLaunchKernelGGL((stft_batch_dispatch_kernel<LOG_M, V>), dim3(grid), dim3(C::WG), 0, s,
-                               static_cast<const char*>(blk), (uint32_t)b.header_off);
+            if (grid != b.ntiles)
+                return hipErrorInvalidValue;
+            hipLaunchKernelGGL((stft_batch_dispatch_kernel<LOG_M, V>), dim3(grid), dim3(C::WG), 0, s, b.jobs,
+                               b.tile_job);
         }
         return hipGetLastError();
     });
@@ -1103,24 +1093,6 @@ static hipError_t batch_info_t(int v, BatchClassInfo* info)
         info->max_blocks_per_cu = per_cu;
         return e;
     });
-}
-
-template <int LOG_M>
-static const void* batch_fn_t(int v, bool persistent)
-{
-    const void* fn = nullptr;
-    (void)with_variant<LOG_M>(v, [&](auto vc) {
-        constexpr int V = decltype(vc)::value;
-        using C = Cfg<LOG_M, V>;
-        if constexpr (C::SHAPE == 0) {
-            fn = persistent ? reinterpret_cast<const void*>(&stft_batch_kernel<LOG_M, C::PLAN>)
-                            : reinterpret_cast<const void*>(&stft_batch_dispatch_kernel<LOG_M, V>);
-        } else {
-            fn = persistent ? nullptr : reinterpret_cast<const void*>(&stft_batch_dispatch_kernel<LOG_M, V>);
-        }
-        return hipSuccess;
-    });
-    return fn;
 }
 
 bool fused_supported(int log_m) { return log_m >= 5 && log_m <= 14; }
@@ -1177,12 +1149,6 @@ hipError_t launch_batch(int log_m, int variant, const BatchClassArgs& b, uint32_
     return with_log_m(log_m, hipErrorInvalidValue, [&](auto lc) {
         return launch_batch_t<decltype(lc)::value>(variant, b, grid, persistent, s);
     });
-}
-
-const void* batch_kernel_fn(int log_m, int variant, bool persistent)
-{
-    return with_log_m(log_m, (const void*)nullptr,
-                      [&](auto lc) { return batch_fn_t<decltype(lc)::value>(variant, persistent); });
 }
 
 hipError_t batch_class_info(int log_m, int variant, BatchClassInfo* info)

@@ -414,8 +414,6 @@ int ostft_server_create(int32_t device, const ostft_server_config* config, ostft
     ostft_server_config cfg{};
     if (config)
         cfg = *config;
-    else
-        cfg.use_graphs = 1;
     if (cfg.arena_bytes == 0)
         cfg.arena_bytes = 1ull << 30;
     if (cfg.max_batch == 0)
@@ -449,8 +447,6 @@ int ostft_server_create(int32_t device, const ostft_server_config* config, ostft
         if (e == hipSuccess)
             e = hipMemcpy(s->arena_h, s->arena_d, cfg.arena_bytes, hipMemcpyDeviceToHost);
     }
-    if (e == hipSuccess)
-        rc = ostft_batch_config(s->ctx, 0, 0, cfg.use_graphs ? 1 : 0, nullptr);
     if (e == hipSuccess && rc == OSTFT_OK && cfg.autotune) {
         for (int exp = 6; exp <= 15 && rc == OSTFT_OK; ++exp)
             rc = ostft_autotune_batch(s->ctx, exp, cfg.autotune_samples ? cfg.autotune_samples : 1ull << 26,
