@@ -85,6 +85,26 @@ hipError_t Scratch::handoff(hipStream_t s)
     return e;
 }
 
+hipError_t Scratch::fork_side(hipStream_t s)
+{
+    hipError_t e = hipSuccess;
+    if (!fork)
+        e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
+    if (e == hipSuccess && !join)
+        e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
+    if (e == hipSuccess && !side)
+        e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
+    if (e == hipSuccess)
+        e = hipEventRecord(fork, s);
+    return e == hipSuccess ? hipStreamWaitEvent(side, fork, 0) : e;
+}
+
+hipError_t Scratch::join_side(hipStream_t s)
+{
+    const hipError_t e = hipEventRecord(join, side);
+    return e == hipSuccess ? hipStreamWaitEvent(s, join, 0) : e;
+}
+
 void Scratch::release()
 {
     if (a) {
@@ -101,9 +121,14 @@ void Scratch::release()
 void Scratch::destroy()
 {
     release();
-    if (done)
-        (void)hipEventDestroy(done);
-    done = nullptr;
+    for (hipEvent_t* e : {&done, &fork, &join}) {
+        if (*e)
+            (void)hipEventDestroy(*e);
+        *e = nullptr;
+    }
+    if (side)
+        (void)hipStreamDestroy(side);
+    side = nullptr;
     used = false;
 }
 
@@ -496,38 +521,61 @@ int pass_tables(ostft_ctx* ctx, int log_m, bool noalloc, PassTables* t)
     return rc;
 }
 
-// Frames of the next chunk with `left` frames to go and room for `cap`.  A
-// chunk of 768 workgroups (96 MiB of scratch) is still in the 256 MB memory-side
-// cache when the last pass reads it; what is left over joins the last chunk or
-// makes one of at least half the size, so that no launch is nearly empty.
-// Scratch of 64 / 96 / 128 / 256 / 1024 MiB, 2^26 samples, 75%, default layout:
-// window 2^17 894 / 848 / 866 / 997 / 892 us, 2^20 990 / 961 / 1011 / 1178 / 1154.
-constexpr uint64_t CHUNK_VALUES = (uint64_t)768 * 16384;
-uint64_t chunk_frames(uint64_t left, uint64_t cap, int log_m)
+// Frames go through both passes a chunk at a time, so that the last pass reads
+// scratch that is still in the 256 MB memory-side cache.  One chunk at a time:
+// 768 workgroups (96 MiB of scratch), what is left over joins the last chunk or
+// makes one of at least half the size.  Requests of more than 2048 workgroups a
+// pass run two chunks of 512 (one round of the GPU) at a time, every other one on
+// a side stream: the last workgroups of one chunk's launch leave the GPU to the
+// other chunk's, and one's loads meet the other's transforms.
+// One / two at a time, overlap 0.5, power: 2^17, 1400 workgroups 144 / 143 us, 2048
+// 209 / 202, 3000 294 / 271; 2^20 153 / 148, 224 / 216, 318 / 287 (below 1024 the fork
+// and join of the streams cost 10-20 us more than they give).  Scratch of one
+// chunk at a time of 64 / 96 / 128 / 256 / 1024 MiB, 2^26 samples, 75%, default
+// layout: 2^17 894 / 848 / 866 / 997 / 892 us; two at a time of 48 / 64 / 80 / 96 MiB each:
+// 805 / 773 / 863 / 890.
+struct Chunks {
+    uint64_t want;  // frames
+    bool two;       // two at a time
+};
+Chunks chunks_of(uint64_t frames, uint64_t room, int log_m, int out_mode)
 {
-    const uint64_t want = CHUNK_VALUES >> log_m;
-    if (cap < want + want / 2) {  // a small budget: equal chunks
+    const uint64_t values = frames << log_m, tile = 16384;
+    // the complex layout writes 16 bytes a value, which at 2^19 and 2^20 push the
+    // second chunk's scratch out of the cache: 577 / 600 and 625 / 673 us (2^18 589 / 576)
+    const bool wide = out_mode == OUT_HALF_COMPLEX && log_m >= 18;
+    Chunks c;
+    c.two = values > 2048 * tile && room >= 2 * ((512 * tile) >> log_m) && !wide;
+    c.want = ((c.two ? 512 : 768) * tile) >> log_m;
+    return c;
+}
+// the most frames of one chunk
+uint64_t chunk_most(const Chunks& c, uint64_t frames) { return std::min(c.two ? c.want : c.want + c.want / 2, frames); }
+// frames of the next chunk with `left` to go and scratch for `cap`
+uint64_t chunk_frames(const Chunks& c, uint64_t left, uint64_t cap)
+{
+    if (cap < std::min(chunk_most(c, left), left)) {  // a small budget: equal chunks
         const uint64_t n = (left + cap - 1) / cap;
-        return n ? (left + n - 1) / n : 1;
+        return (left + n - 1) / n;
     }
-    return left <= want + want / 2 ? left : want;
+    if (c.two)
+        return left <= c.want ? left : left < 2 * c.want ? (left + 1) / 2 : c.want;
+    return left <= c.want + c.want / 2 ? left : c.want;
 }
 
-// Both passes over the request's frames, a chunk at a time through `buf`
-// (`cap` frames).
+// Both passes over the request's frames, chunk by chunk through `buf` (`cap`
+// frames; two such buffers with `sc`, whose side stream takes every other chunk).
 int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& t, float2* buf, uint64_t cap,
-               hipStream_t s)
+               const Chunks& c, hipStream_t s, Scratch* sc = nullptr)
 {
     PassArgs p;
     p.sig = a.in;
     p.L = a.L;
     p.hop = a.hop;
     p.win = a.win;
-    p.dst = buf;
     p.tw_r = t.r0;
 
     LastArgs la;
-    la.src = buf;
     la.tw_r = t.r1;
     la.tw_n = a.tw_n;
     std::copy(std::begin(t.k), std::end(t.k), la.tw_k);
@@ -537,14 +585,23 @@ int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& 
     la.out_mode = a.out_mode;
     la.dc = a.dc;
 
-    for (uint64_t f0 = 0; f0 < a.frames; f0 = p.frames) {
+    hipError_t e = sc ? sc->fork_side(s) : hipSuccess;
+    if (e != hipSuccess)
+        return ctx_hip_fail(ctx, e, "multi-pass side stream");
+    uint32_t i = 0;
+    for (uint64_t f0 = 0; e == hipSuccess && f0 < a.frames; f0 = p.frames, ++i) {
+        const bool side = sc && (i & 1u);
+        p.dst = buf + (side ? cap << log_m : 0);
+        la.src = p.dst;
         p.frame0 = la.frame0 = f0;
-        p.frames = la.frames = f0 + chunk_frames(a.frames - f0, cap, log_m);
-        const hipError_t e = launch_passes(log_m, p, la, s);
-        if (e != hipSuccess)
-            return ctx_hip_fail(ctx, e, "multi-pass launch");
+        p.frames = la.frames = f0 + chunk_frames(c, a.frames - f0, cap);
+        e = launch_passes(log_m, p, la, side ? sc->side : s);
     }
-    return OSTFT_OK;
+    if (sc) {  // also after a failed launch: what follows on s comes after the side stream's work
+        const hipError_t j = sc->join_side(s);
+        e = e == hipSuccess ? j : e;
+    }
+    return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "multi-pass launch");
 }
 
 // Scratch of the allocation-free entry point: a fixed device array, one
@@ -588,9 +645,10 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     // chain (acquire / handoff) orders their GPU work across streams
     std::lock_guard<std::mutex> lk(ctx_scratch_mutex(ctx));
     Scratch& sc = ctx_scratch(ctx);
-    const uint64_t most = (CHUNK_VALUES + CHUNK_VALUES / 2) >> log_m;  // of any chunk
-    const uint64_t cap = std::min(std::min(multipass_chunk_frames(sc.budget, log_m), most), a.frames);
-    hipError_t e = sc.ensure(cap * M);
+    const uint64_t room = multipass_chunk_frames(sc.budget, log_m);
+    const Chunks c = chunks_of(a.frames, room, log_m, a.out_mode);
+    const uint64_t cap = std::min(room, chunk_most(c, a.frames));
+    hipError_t e = sc.ensure((c.two ? 2 : 1) * cap * M);
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass scratch allocation");
     e = sc.acquire(s);
@@ -599,7 +657,7 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     PassTables t;
     int rc = pass_tables(ctx, log_m, false, &t);
     if (rc == OSTFT_OK)
-        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, s);
+        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, c, s, c.two ? &sc : nullptr);
     if (rc != OSTFT_OK)
         return rc;
     e = sc.handoff(s);
@@ -627,7 +685,8 @@ int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs&
     const int rc = pass_tables(ctx, log_m, true, &t);
     if (rc != OSTFT_OK)
         return rc;
-    return run_chunks(ctx, log_m, a, t, buf, STATIC_SCRATCH_BYTES / frame_bytes, s);
+    Chunks c = chunks_of(a.frames, 0, log_m, a.out_mode);  // no other stream, no event
+    return run_chunks(ctx, log_m, a, t, buf, std::min(STATIC_SCRATCH_BYTES / frame_bytes, a.frames), c, s);
 }
 
 }  // namespace ostft

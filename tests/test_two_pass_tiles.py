@@ -28,6 +28,9 @@ LAYOUTS = {"": po.OUT_COMPAT_POWER, "--magnitude_return": po.OUT_MAGNITUDE,
 
 @pytest.fixture(scope="module")
 def runner():
+    import torch  # ahead of the engine library, which then shares its HIP runtime
+
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
     r = ostft.Runner(0)
     yield r
     r.close()
@@ -76,3 +79,31 @@ def test_long_request_equals_its_frames_alone(runner, exp, frames):
         for f in sorted({0, 1, count // 3, count // 2, count - 2, count - 1}):
             alone = runner.run_device(x[f * hop: f * hop + n].contiguous(), p)
             assert torch.equal(y[f * per: (f + 1) * per], alone[:per]), (exp, layout, f)
+
+
+def test_captured_long_request_replays(runner):
+    """Two chunks at a time fork to a side stream and join again: also inside a
+    captured graph, whose replays follow new inputs and eager work between."""
+    import torch
+
+    exp, frames = 17, 620  # 2480 workgroups a pass
+    n = 1 << exp
+    x = torch.zeros((frames - 1) * (n // 4) + n, device="cuda")
+    p = ostft.parse_options("--hanning_window --power_return", exp, 0.75)
+    out = torch.empty(ostft.geometry(p, x.numel())["out_floats"], device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        runner.run_device(x, p, out=out)  # tables and scratch become resident
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        runner.run_device(x, p, out=out)
+    with torch.cuda.stream(s):
+        for rep in range(3):
+            x.normal_(generator=torch.Generator("cuda").manual_seed(rep))
+            out.zero_()
+            g.replay()
+            got = out.clone()
+            want = runner.run_device(x, p)
+            s.synchronize()
+            assert torch.equal(got, want), rep

@@ -27,6 +27,9 @@ LAYOUTS = {"": (po.OUT_COMPAT_POWER, N_), "--magnitude_return": (po.OUT_MAGNITUD
 
 @pytest.fixture(scope="module")
 def runner():
+    import torch  # ahead of the engine library, which then shares its HIP runtime
+
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
     r = ostft.Runner(0)
     yield r
     r.close()
