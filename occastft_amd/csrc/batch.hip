@@ -29,6 +29,7 @@
 
 #include "batch.hpp"
 #include "multipass.hpp"
+#include "side_stream.hpp"
 
 namespace ostft {
 
@@ -36,6 +37,8 @@ namespace {
 
 constexpr int LOG_M_MIN = 5, LOG_M_MAX = 14, NCLS = LOG_M_MAX - LOG_M_MIN + 1;
 constexpr size_t ALIGN = 256;
+// batches from so many tiles, and so many a request, use two streams (run_batch)
+constexpr uint64_t SIDE_TILES = 32768, SIDE_TILES_PER_REQUEST = 64;
 
 size_t align_up(size_t x) { return (x + ALIGN - 1) & ~(ALIGN - 1); }
 
@@ -71,6 +74,7 @@ struct BatchState {
     int shape[NCLS] = {};       // workgroup shape (engine variant / 4); persistent needs 0
     int plan_override[NCLS];    // >= 0: radix plan for this class instead of the context's (autotuning)
     int variant[NCLS] = {};     // engine variant of each class in the current batch
+    SideStream side;
     BatchClassInfo info[NCLS][FUSED_VARIANTS] = {};
     bool info_ok[NCLS][FUSED_VARIANTS] = {};
 
@@ -301,15 +305,31 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         hipLaunchKernelGGL(batch_fill_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj, tj,
                            counters);
         e = hipGetLastError();
+        // A large batch runs its classes on two streams in turn: the last tiles of
+        // one class leave the GPU to the other stream's.  256 mixed requests
+        // (47762 tiles of six classes): 470 -> 441 us (454 with each class on the
+        // stream with fewer tiles so far); the fork and join cost the host 20 us, more than a smaller batch
+        // gains (256 requests of 12000 tiles 220 -> 258 us).
+        const bool two = total >= SIDE_TILES && total >= SIDE_TILES_PER_REQUEST * nreq && __builtin_popcount(mask) > 1;
+        if (e == hipSuccess && two)
+            e = st->side.fork(s);
+        const bool forked = e == hipSuccess && two;
+        int turn = 0;
         for (int c = 0; e == hipSuccess && c < NCLS; ++c) {
             if (!(mask >> c & 1u))
                 continue;
+            const bool side = two && (turn++ & 1);
             BatchClassArgs a;
             a.jobs = bj + first_job[c];
             a.tile_job = tj + first_tile[c];
             a.counter = counters + c;
             a.ntiles = (uint32_t)ntiles[c];
-            e = launch_batch(c + LOG_M_MIN, st->variant[c], a, class_grid(st, c, ntiles[c]), st->persistent[c] != 0, s);
+            e = launch_batch(c + LOG_M_MIN, st->variant[c], a, class_grid(st, c, ntiles[c]), st->persistent[c] != 0,
+                             side ? st->side.stream : s);
+        }
+        if (forked) {  // also after a failed launch: what follows on s comes after the side stream's work
+            const hipError_t j = st->side.join(s);
+            e = e == hipSuccess ? j : e;
         }
         if (e == hipSuccess)
             e = hipEventRecord(sl.done, s);
@@ -631,6 +651,7 @@ void batch_release(ostft_ctx* ctx)
         if (sl.done)
             (void)hipEventDestroy(sl.done);
     }
+    b->side.destroy();
     delete b;
     b = nullptr;
 }

@@ -85,26 +85,6 @@ hipError_t Scratch::handoff(hipStream_t s)
     return e;
 }
 
-hipError_t Scratch::fork_side(hipStream_t s)
-{
-    hipError_t e = hipSuccess;
-    if (!fork)
-        e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
-    if (e == hipSuccess && !join)
-        e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
-    if (e == hipSuccess && !side)
-        e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
-    if (e == hipSuccess)
-        e = hipEventRecord(fork, s);
-    return e == hipSuccess ? hipStreamWaitEvent(side, fork, 0) : e;
-}
-
-hipError_t Scratch::join_side(hipStream_t s)
-{
-    const hipError_t e = hipEventRecord(join, side);
-    return e == hipSuccess ? hipStreamWaitEvent(s, join, 0) : e;
-}
-
 void Scratch::release()
 {
     if (a) {
@@ -121,14 +101,10 @@ void Scratch::release()
 void Scratch::destroy()
 {
     release();
-    for (hipEvent_t* e : {&done, &fork, &join}) {
-        if (*e)
-            (void)hipEventDestroy(*e);
-        *e = nullptr;
-    }
-    if (side)
-        (void)hipStreamDestroy(side);
-    side = nullptr;
+    if (done)
+        (void)hipEventDestroy(done);
+    done = nullptr;
+    side.destroy();
     used = false;
 }
 
@@ -585,7 +561,7 @@ int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& 
     la.out_mode = a.out_mode;
     la.dc = a.dc;
 
-    hipError_t e = sc ? sc->fork_side(s) : hipSuccess;
+    hipError_t e = sc ? sc->side.fork(s) : hipSuccess;
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass side stream");
     uint32_t i = 0;
@@ -595,10 +571,10 @@ int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& 
         la.src = p.dst;
         p.frame0 = la.frame0 = f0;
         p.frames = la.frames = f0 + chunk_frames(c, a.frames - f0, cap);
-        e = launch_passes(log_m, p, la, side ? sc->side : s);
+        e = launch_passes(log_m, p, la, side ? sc->side.stream : s);
     }
     if (sc) {  // also after a failed launch: what follows on s comes after the side stream's work
-        const hipError_t j = sc->join_side(s);
+        const hipError_t j = sc->side.join(s);
         e = e == hipSuccess ? j : e;
     }
     return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "multi-pass launch");

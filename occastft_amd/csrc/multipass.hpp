@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "engine.hpp"
+#include "side_stream.hpp"
 
 struct ostft_ctx;
 
@@ -18,15 +19,12 @@ struct Scratch {
     uint64_t cap = 0;                      // complex elements
     uint64_t budget = (uint64_t)1 << 30;  // bytes per chunk of frames
     hipEvent_t done = nullptr;             // recorded after the last call's launches
-    hipStream_t side = nullptr;            // every other chunk of a long request runs here
-    hipEvent_t fork = nullptr, join = nullptr;
+    SideStream side;                       // every other chunk of a long request runs here
     hipStream_t last = nullptr;            // the stream of that call
     bool used = false;
     hipError_t ensure(uint64_t n);
     hipError_t acquire(hipStream_t s);  // order stream s after the previous user
     hipError_t handoff(hipStream_t s);  // record the end of this call's launches
-    hipError_t fork_side(hipStream_t s);  // `side` follows what s holds so far
-    hipError_t join_side(hipStream_t s);  // s follows what `side` holds so far
     void release();                     // frees the buffer (after the last user's launches)
     void destroy();                     // release + the event
 };
