@@ -145,8 +145,8 @@ uint32_t class_grid(const BatchState* st, int c, uint64_t ntiles)
 // tile table, and its record.
 constexpr int FILL_THREADS = 256;
 __global__ void __launch_bounds__(FILL_THREADS)
-    batch_fill_kernel(const BatchUpload* __restrict__ up, BatchJob* __restrict__ jobs, uint32_t* __restrict__ tiles,
-                      uint32_t* __restrict__ counters)
+    stft_batch_table_kernel(const BatchUpload* __restrict__ up, BatchJob* __restrict__ jobs,
+                            uint32_t* __restrict__ tiles, uint32_t* __restrict__ counters)
 {
     const uint32_t j = blockIdx.x, tid = threadIdx.x;
     const BatchUpload* u = up + j;
@@ -302,8 +302,8 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         BatchJob* const bj = reinterpret_cast<BatchJob*>(sl.d + jobs_off);
         uint32_t* const tj = reinterpret_cast<uint32_t*>(sl.d + tiles_off);
         const uint32_t parts = (uint32_t)std::min<uint64_t>(1 + most / (16 * FILL_THREADS), 256);
-        hipLaunchKernelGGL(batch_fill_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj, tj,
-                           counters);
+        hipLaunchKernelGGL(stft_batch_table_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj,
+                           tj, counters);
         e = hipGetLastError();
         // A large batch runs its classes on two streams in turn: the last tiles of
         // one class leave the GPU to the other stream's.  256 mixed requests
