@@ -266,10 +266,10 @@ int ostft_autotune_batch(ostft_ctx* ctx, int32_t exp, uint64_t samples, const os
                          int32_t* best_blocks_per_cu, int32_t* best_shape, int32_t* best_plan, double* best_ms);
 
 /* Scratch budget of the two-pass path (windows 2^17..2^20), in bytes: its
- * frames go through both passes in chunks whose intermediate spectra fit the
- * budget (at least one frame per chunk).  bytes = 0 leaves it; a budget below
- * the scratch already held frees that scratch.  *current (may be NULL)
- * receives the budget in force.  Default 1 GiB.  No counterpart in the
+ * frames go through both passes in chunks, and the intermediate spectra of the
+ * chunks in work fit the budget (one frame always does).  bytes = 0 leaves
+ * it; a budget below the scratch already held frees that scratch.  *current
+ * (may be NULL) receives the budget in force.  Default 1 GiB.  No counterpart in the
  * reference, whose runners hold whole-signal intermediate buffers. */
 int ostft_scratch_budget(ostft_ctx* ctx, uint64_t bytes, uint64_t* current);
 

@@ -594,8 +594,6 @@ float2* static_ptr[MAX_DEVICES] = {};
 
 }  // namespace
 
-uint64_t multipass_static_scratch_bytes() { return STATIC_SCRATCH_BYTES; }
-
 hipError_t multipass_static_scratch_init(int device)
 {
     if (device < 0 || device >= MAX_DEVICES)

@@ -17,7 +17,7 @@ namespace ostft {
 struct Scratch {
     float2* a = nullptr;
     uint64_t cap = 0;                      // complex elements
-    uint64_t budget = (uint64_t)1 << 30;  // bytes per chunk of frames
+    uint64_t budget = (uint64_t)1 << 30;  // bytes it may take
     hipEvent_t done = nullptr;             // recorded after the last call's launches
     SideStream side;                       // every other chunk of a long request runs here
     hipStream_t last = nullptr;            // the stream of that call
@@ -43,10 +43,9 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
 int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs& a, hipStream_t s);
 // Looks up the fixed scratch of the current device, `device` (once per device).
 hipError_t multipass_static_scratch_init(int device);
-uint64_t multipass_static_scratch_bytes();
 
-// Frames per chunk (both passes run a chunk before the next one starts):
-// as many as fit `budget` bytes of scratch, at least one.
+// Frames whose scratch fits `budget` bytes, at least one: the most that are
+// between the two passes at any time.
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m);
 
 bool multipass_supported(int log_m);  // complex sizes 2^16 .. 2^19

@@ -1,5 +1,5 @@
-// stockham.hpp -- the LDS-exchanged Stockham engine shared by the fused
-// single-kernel path and the multi-pass column kernels.
+// stockham.hpp -- the LDS-exchanged Stockham engine of the fused
+// single-kernel path (windows 2^6..2^15).
 //
 // A "group" of T = M/VPT threads owns one complex transform of size
 // M = 2^LOG_M with VPT = 16 (or 8) values per thread in VGPRs.  Passes are
