@@ -18,8 +18,8 @@ reported beside it as `qtconst_frames_per_s`.
 Sub-objects of the same JSON line (each with roofline, traffic, cpu_baseline):
   large  -- 2^27-sample signal (N(0,1) noise + 0.5-amplitude linear chirp
             0 -> 0.5 cycles/sample), windows 2^16..2^20, overlap 0 and 75%,
-            Blackman + DC removal, power spectrum (N/2+1 bins): the two-pass
-            path; 10 requests per step.
+            Blackman + DC removal, power spectrum (N/2+1 bins): one kernel at
+            2^16, two passes above; 10 requests per step.
   batch  -- 4096 signals of 2^18 samples of unit-variance 1/f (pink) noise,
             windows 64, 256, 1024, overlap 50%, Hanning, complex half
             spectrum, in four forms (FP32 through the ragged tile queue, FP32
@@ -526,7 +526,7 @@ def bench_large(args, runner) -> dict:
     cold_ms = cold_time(lambda: runner.run_device(x, p, out=out, stream=stream), stream, max(3, args.steps))
     total_bytes = sum(algorithmic_bytes(g, 1 << e) for e, ov, p, g in reqs)
     res = header(args, frames / (ms_per_step / 1e3), "frames/s", ms_per_step, {
-        "workload": "plain FP32 large-window two-pass path: 2^27-sample signal (N(0,1) + 0.5 linear chirp "
+        "workload": "plain FP32 large windows: 2^27-sample signal (N(0,1) + 0.5 linear chirp "
                     "0->0.5 cycles/sample), windows 2^16..2^20, overlap 0/75%, Blackman + DC removal, power "
                     "spectrum N/2+1 bins (10 requests per step)",
         "signal_samples": LARGE_LEN, "requests_per_step": len(reqs), "frames_per_step": frames})
