@@ -256,6 +256,17 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
     for (int c = 0; c < NCLS; ++c)
         if (ntiles[c] >= 0x7fffffffull - 2ull * (uint64_t)st->cu_count * 64u)  // grid limit; claims overrun by <= 2/workgroup
             return ctx_fail(ctx, OSTFT_ERR_TOO_LARGE, "more than 2^31 tiles of one window size in a batch");
+    if (__builtin_popcount(mask) >= 3) {
+        // A captured batch replays from records that the next batch but one
+        // rewrites.  Batches of one or two window sizes may be captured by a caller
+        // who sees to that; with more it is refused.
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        const hipError_t e = hipStreamIsCapturing(s, &cs);
+        if (e != hipSuccess)
+            return ctx_hip_fail(ctx, e, "batch stream");
+        if (cs != hipStreamCaptureStatusNone)
+            return ctx_fail(ctx, OSTFT_ERR_UNSUPPORTED, "a batch of three or more window sizes cannot be captured");
+    }
     if (mask) {
         // 3. descriptor block layout: claim counters, requests class by class,
         //    tile tables class by class
