@@ -342,11 +342,12 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
             const hipError_t j = st->side.join(s);
             e = e == hipSuccess ? j : e;
         }
-        if (e == hipSuccess)
-            e = hipEventRecord(sl.done, s);
+        // also after a failed launch: what was queued may still read this slot
+        const hipError_t r = hipEventRecord(sl.done, s);
+        sl.used = sl.used || r == hipSuccess;
+        e = e == hipSuccess ? r : e;
         if (e != hipSuccess)
             return ctx_hip_fail(ctx, e, "batch launch");
-        sl.used = true;
     }
     for (uint32_t i : mfma) {
         const int xf = (jobs[i].params.flags & OSTFT_FLAG_MFMA_FP16) ? XF_MFMA_FP16 : XF_MFMA_BF16;

@@ -632,9 +632,10 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     int rc = pass_tables(ctx, log_m, false, &t);
     if (rc == OSTFT_OK)
         rc = run_chunks(ctx, log_m, a, t, sc.a, cap, c, s, c.two ? &sc : nullptr);
+    // also after a failed launch: what was queued may still use the scratch
+    e = sc.handoff(s);
     if (rc != OSTFT_OK)
         return rc;
-    e = sc.handoff(s);
     return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "multi-pass scratch event");
 }
 
