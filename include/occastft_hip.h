@@ -165,7 +165,7 @@ int ostft_run_device(ostft_ctx* ctx, const ostft_params* params, const float* d_
  *     event.  Every call on a GPU shares that array and it keeps the last
  *     call's contents (each call overwrites what it reads first): calls that
  *     overlap in time on one GPU race; keep them on one stream or ordered.
- * Windows up to 2^16 use no scratch. */
+ * Windows up to 2^16 use no scratch here. */
 int ostft_run_device_noalloc(ostft_ctx* ctx, const ostft_params* params, const float* d_in,
                              uint64_t full_size, float* d_out, uint64_t out_cap, void* hip_stream);
 
@@ -267,7 +267,8 @@ int ostft_engine_variant(ostft_ctx* ctx, int32_t exp, int32_t shape, int32_t pla
 int ostft_autotune_batch(ostft_ctx* ctx, int32_t exp, uint64_t samples, const ostft_params* like,
                          int32_t* best_blocks_per_cu, int32_t* best_shape, int32_t* best_plan, double* best_ms);
 
-/* Scratch budget of the two-pass path (windows 2^17..2^20), in bytes: its
+/* Scratch budget of the two-pass path (windows 2^17..2^20, and requests of few
+ * frames at 2^16 where the budget holds them), in bytes: its
  * frames go through both passes in chunks, and the intermediate spectra of the
  * chunks in work fit the budget (one frame always does).  bytes = 0 leaves
  * it; a budget below the scratch already held frees that scratch.  *current

@@ -14,7 +14,7 @@
 // longer for every mix, 58 against 35 us a batch of 24 requests of three sizes, 280
 // against 274 us one of 256 requests of ten.
 //
-// Requests of windows >= 2^16 (one launch, or the two-pass path) and requests of the matrix-core
+// Requests of windows >= 2^16 (one kernel or two passes) and requests of the matrix-core
 // form run after the tile-queue launches, one request at a time, on the same
 // stream.
 #include <hip/hip_runtime.h>
@@ -356,13 +356,7 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
             return ctx_hip_fail(ctx, e, "batch MFMA launch");
     }
     for (uint32_t i : large) {
-        if (wide_supported(lm[i])) {
-            const hipError_t e = launch_wide(args[i], 1, s);
-            if (e != hipSuccess)
-                return ctx_hip_fail(ctx, e, "batch wide launch");
-            continue;
-        }
-        rc = run_multipass(ctx, lm[i], args[i], s);
+        rc = wide_supported(lm[i]) ? run_wide(ctx, lm[i], args[i], s) : run_multipass(ctx, lm[i], args[i], s);
         if (rc != OSTFT_OK)
             return rc;
     }

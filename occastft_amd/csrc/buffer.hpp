@@ -21,6 +21,12 @@ __device__ __forceinline__ float2 load2(__amdgpu_buffer_rsrc_t r, uint32_t lane_
 {
     return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, off, 0));
 }
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ float4 load4(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off)
+{
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, off, 0));
+}
 __device__ __forceinline__ void store1(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t off, float v)
 {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, lane_off, off, 0);

@@ -657,10 +657,8 @@ int run_device_geometry(ostft_ctx* ctx, const ostft_params* params, const float*
             return hip_fail(ctx, e, "fused STFT launch");
         return OSTFT_OK;
     }
-    if (ostft::wide_supported(log_m)) {
-        const hipError_t e = ostft::launch_wide(a, 1, s);
-        return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "wide STFT launch");
-    }
+    if (ostft::wide_supported(log_m))
+        return ostft::run_wide(ctx, log_m, a, s);
     return ostft::run_multipass(ctx, log_m, a, s);
 }
 }  // namespace
@@ -729,7 +727,7 @@ int ostft_run_strided_device(ostft_ctx* ctx, const ostft_params* params, const f
         return OSTFT_OK;
     a.in_stride = in_stride;
     a.out_stride = out_stride;
-    if (ostft::fused_supported(log_m) || ostft::wide_supported(log_m)) {
+    if (ostft::fused_supported(log_m) || (ostft::wide_supported(log_m) && count > 1)) {
         for (uint32_t y0 = 0; y0 < count; y0 += 65535u) {  // grid.y limit
             ostft::FusedArgs ay = a;
             ay.in = d_in + (uint64_t)y0 * in_stride;
@@ -747,7 +745,8 @@ int ostft_run_strided_device(ostft_ctx* ctx, const ostft_params* params, const f
         ay.in = d_in + (uint64_t)y * in_stride;
         ay.out = d_out + (uint64_t)y * out_stride;
         ay.in_stride = ay.out_stride = 0;
-        const int r = ostft::run_multipass(ctx, log_m, ay, s);
+        const int r = ostft::wide_supported(log_m) ? ostft::run_wide(ctx, log_m, ay, s)
+                                                   : ostft::run_multipass(ctx, log_m, ay, s);
         if (r != OSTFT_OK)
             return r;
     }

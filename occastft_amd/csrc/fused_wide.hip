@@ -18,6 +18,8 @@
 // 4.4 without the transforms, 3.8 without the exchanges, 4.0 without the
 // stores.  A persistent grid that loads the next frame while this one's result
 // goes out took 850 us (a wave's loads wait for the stores issued before them).
+// Requests of few frames, which leave most CUs idle here, go through the two
+// passes (run_wide in multipass.hip).
 #include "buffer.hpp"
 #include "engine.hpp"
 #include "epilogue.hpp"

@@ -1,5 +1,5 @@
 // multipass.hip -- STFT for complex transform sizes M = 2^16 .. 2^19
-// (windows 2^17 .. 2^20).
+// (windows 2^17 .. 2^20), and 2^15 (window 2^16) where a request has few frames.
 //
 // Same pipeline as the fused kernel (gather + window, FFT, split epilogue),
 // but the transform fits no workgroup's registers, so it is cut into two
@@ -7,8 +7,8 @@
 // EXP separate radix-2 StockHamCommon launches of OKL/EXPCommon.okl:194-245,
 // one per stage, and the separate ToPower / toHalfComplexFormat passes).
 //
-// Both passes hold 32 complex values a thread in registers, 16384 or 8192 a
-// workgroup, as R-point transforms of as many columns, and take a column in two
+// Both passes hold 32 complex values a thread in registers, 16384, 8192 or
+// 4096 a workgroup, as R-point transforms of as many columns, and take a column in two
 // register steps of fused multiply-add butterflies (twisted_dft.hpp) with one
 // exchange between them, whose real and imaginary parts go through LDS in turn.
 //   * first pass (R0 = 2^10 = 32 x 32): samples come from the signal (overlap
@@ -32,7 +32,7 @@
 // window 2^18, overlap 0, default layout 594 -> 507 us (2.15 GB moved, 4.2 TB/s; a
 // plain copy of 2 GiB runs at 4.9); 2^20, 75%, power 2050 -> 1590 us; 2^26
 // samples, 75%, default layout: 2^17 853 -> 839, 2^18 987 -> 878, 2^19 1040 -> 903,
-// 2^20 1239 -> 961 us; one frame: 20-26 -> 18-22 us.
+// 2^20 1239 -> 961 us; one frame: 20-26 -> 15-20 us.
 #include "../../include/occastft_hip.h"
 
 #include <algorithm>
@@ -108,15 +108,17 @@ void Scratch::destroy()
     used = false;
 }
 
-// The split M = R0 x R1: R0 = 2^10 = 32 x 32, R1 = 2^6 .. 2^9 = R1/16 x 16
+// The split M = R0 x R1: R0 = 2^10 = 32 x 32, R1 = 2^6 .. 2^9 = R1/16 x 16 (32 in one
+// step for window 2^16)
 constexpr int MP_LOG_R0 = 10, MP_R0 = 1 << MP_LOG_R0;
 // Scratch of a frame is [g / 16][k][g mod 16] for butterfly g and result k of
 // the first pass: a run of 16 values is a cache line and a quarter wave.
 constexpr uint32_t MP_RUN = 16;
 
 // A workgroup's threads and complex values.  512 threads: two workgroups a CU
-// and longer runs in memory; 256 threads: twice the workgroups, for requests
-// that leave CUs idle otherwise.  A frame's arithmetic is the same in both.
+// and longer runs in memory; 256 and 128 threads: two and four times the
+// workgroups, for requests that leave CUs idle otherwise.  A frame's arithmetic
+// is the same in all.
 template <int THREADS>
 struct Tile {
     static constexpr uint32_t ELEMS = 32 * THREADS;
@@ -149,7 +151,7 @@ __device__ __forceinline__ void gather_step(float2 (&v)[32], const float* rd)
     });
 }
 
-// First pass: C = 16 (8 with 256 threads) butterflies g of one frame (columns),
+// First pass: C = 16 (8 with 256 threads, 4 with 128) butterflies g of one frame (columns),
 // lanes along the columns: the samples come straight into the butterflies'
 // registers and the results leave from them, in runs of C values either way.
 template <int LOG_M, int THREADS>
@@ -279,54 +281,69 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
         const uint32_t k = b * CB + (c & (CB - 1));
         return c < CB ? k : k == 0 ? Ns / 2 : Ns - k;
     };
-    // inputs g = t + 16 j of butterfly k: scratch [j][k][t]; columns cg + CSTEP i
     float2 v[32];
-    {
-        const uint32_t t = tid & 15u, cg = tid >> 4;
-        const auto bs = buffer(a.src + (P - a.frame0) * M, 8 * M);
-        cfor<0, NC>([&](auto i) {
-            const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
-            cfor<0, r1>([&](auto j) {
-                v[decltype(i)::value * r1 + decltype(j)::value] =
-                    load2(bs, 8 * (k * MP_RUN + t), 8 * Ns * MP_RUN * decltype(j)::value);
-            });
-        });
-        float* const wr = lds + (r1 * C + PAD) * t + cg;
-        cfor<0, NC>([&](auto i) {
-            // twist over j: W_M^(16 k)
-            constexpr int O = decltype(i)::value * r1;
-            const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
-            Twist<r1> tw;
-            cfor<0, ilog2(r1)>([&](auto l) {
-                tw.base[decltype(l)::value] = a.tw_k[4 + ilog2(r1) - 1 - decltype(l)::value][k];
-            });
-            twisted_dft<r1, O, 1, true>(v, tw);
-            cfor<0, r1>([&](auto q) { wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[O + decltype(q)::value].x; });
-        });
-        const float* const rd = lds + tid;
-        __syncthreads();
-        gather_step<C, r1, PAD, T, 2, 0>(v, rd);
-        __syncthreads();
-        cfor<0, NC>([&](auto i) {
-            cfor<0, r1>([&](auto q) {
-                wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[decltype(i)::value * r1 + decltype(q)::value].y;
-            });
-        });
-        __syncthreads();
-        gather_step<C, r1, PAD, T, 2, 1>(v, rd);
-    }
     const uint32_t c = tid % C, t = tid / C, k = butterfly(c);
-    const float2 wt = a.tw_n[k + Ns * t];
-    // second step, butterfly t + T u over 16 inputs: twist W_M^k W_R^(t + T u)
-    cfor<0, 2>([&](auto u) {
-        constexpr int UU = decltype(u)::value;
-        Twist<16> tu;
-        cfor<0, 4>([&](auto l) {
-            constexpr uint32_t J = 3 - decltype(l)::value;
-            tu.base[decltype(l)::value] = cmul(a.tw_k[J][k], a.tw_r[(t + T * UU) << J]);
+    if constexpr (R == 32) {
+        // one step of 32 points: scratch [g / 16][k][g mod 16], the butterfly's
+        // inputs are two runs of its thread
+        const auto bs = buffer(a.src + (P - a.frame0) * M, 8 * M);
+        cfor<0, 16>([&](auto j) {
+            constexpr uint32_t J = decltype(j)::value;
+            const float4 x = load4(bs, 8 * k * MP_RUN, 8 * Ns * MP_RUN * (J / 8) + 16 * (J % 8));
+            v[2 * J] = make_float2(x.x, x.y);
+            v[2 * J + 1] = make_float2(x.z, x.w);
         });
-        twisted_dft<16, UU, 2, true>(v, tu);
-    });
+        Twist<32> tw;
+        cfor<0, 5>([&](auto l) { tw.base[decltype(l)::value] = a.tw_k[4 - decltype(l)::value][k]; });
+        twisted_dft<32, 0, 1, true>(v, tw);
+    } else {
+        // inputs g = t + 16 j of butterfly k: scratch [j][k][t]; columns cg + CSTEP i
+        {
+            const uint32_t t = tid & 15u, cg = tid >> 4;
+            const auto bs = buffer(a.src + (P - a.frame0) * M, 8 * M);
+            cfor<0, NC>([&](auto i) {
+                const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
+                cfor<0, r1>([&](auto j) {
+                    v[decltype(i)::value * r1 + decltype(j)::value] =
+                        load2(bs, 8 * (k * MP_RUN + t), 8 * Ns * MP_RUN * decltype(j)::value);
+                });
+            });
+            float* const wr = lds + (r1 * C + PAD) * t + cg;
+            cfor<0, NC>([&](auto i) {
+                // twist over j: W_M^(16 k)
+                constexpr int O = decltype(i)::value * r1;
+                const uint32_t k = butterfly(cg + CSTEP * decltype(i)::value);
+                Twist<r1> tw;
+                cfor<0, ilog2(r1)>([&](auto l) {
+                    tw.base[decltype(l)::value] = a.tw_k[4 + ilog2(r1) - 1 - decltype(l)::value][k];
+                });
+                twisted_dft<r1, O, 1, true>(v, tw);
+                cfor<0, r1>([&](auto q) { wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[O + decltype(q)::value].x; });
+            });
+            const float* const rd = lds + tid;
+            __syncthreads();
+            gather_step<C, r1, PAD, T, 2, 0>(v, rd);
+            __syncthreads();
+            cfor<0, NC>([&](auto i) {
+                cfor<0, r1>([&](auto q) {
+                    wr[CSTEP * decltype(i)::value + C * decltype(q)::value] = v[decltype(i)::value * r1 + decltype(q)::value].y;
+                });
+            });
+            __syncthreads();
+            gather_step<C, r1, PAD, T, 2, 1>(v, rd);
+        }
+        // second step, butterfly t + T u over 16 inputs: twist W_M^k W_R^(t + T u)
+        cfor<0, 2>([&](auto u) {
+            constexpr int UU = decltype(u)::value;
+            Twist<16> tu;
+            cfor<0, 4>([&](auto l) {
+                constexpr uint32_t J = 3 - decltype(l)::value;
+                tu.base[decltype(l)::value] = cmul(a.tw_k[J][k], a.tw_r[(t + T * UU) << J]);
+            });
+            twisted_dft<16, UU, 2, true>(v, tu);
+        });
+    }
+    const float2 wt = a.tw_n[k + Ns * t];
     // value i is row q = t + T i of column c: Z[k + Ns q]
     const bool k0 = b == 0 && c == 0;
     if (a.dc && k0 && t == 0)  // subtracting the mean only moves Z[0]
@@ -424,11 +441,12 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
 
 namespace {
 
-// f(integral_constant<int, LOG_M>) for a runtime log_m in 16 .. 19
+// f(integral_constant<int, LOG_M>) for a runtime log_m in 15 .. 19
 template <typename F>
 hipError_t with_log_m(int log_m, F&& f)
 {
     switch (log_m) {
+    case 15: return f(std::integral_constant<int, 15>{});
     case 16: return f(std::integral_constant<int, 16>{});
     case 17: return f(std::integral_constant<int, 17>{});
     case 18: return f(std::integral_constant<int, 18>{});
@@ -456,20 +474,34 @@ hipError_t launch_tiles(const PassArgs& p, const LastArgs& la, hipStream_t s)
 // 22.7 / 18.3 us, 16 frames (1.0 M values) 27.2 / 21.5, 64 (4.2 M) 37.3 / 37.4, 128
 // 68.0 / 79.0; 2^20, 4 frames (2.1 M) 31.3 / 29.1, 8 (4.2 M) 39.8 / 42.2, 16 71.7 / 95.7.
 constexpr uint64_t SMALL_VALUES = (uint64_t)192 * 16384;
+// Up to 160 workgroups of 128 threads leave every one a CU of its own.  256 / 128
+// threads, overlap 0, power: 2^16, 5 frames 18.0 / 15.7 us, 20 (0.66 M values) 19.6 /
+// 17.6, 36 20.8 / 23.2; 2^17, 2 frames 16.8 / 15.5, 10 (0.66 M) 18.7 / 18.1, 14 19.4 /
+// 20.3; 2^18, 2 frames 17.3 / 16.0, 4 (0.52 M) 18.1 / 17.2, 7 19.5 / 20.5; 2^19, 2 (0.52
+// M) 18.4 / 17.6, 3 19.3 / 19.4.  At 2^20 their output runs are four values: one
+// frame, complex half, 19.9 / 22.8.
+constexpr uint64_t TINY_VALUES = (uint64_t)160 * 4096;
 
 hipError_t launch_passes(int log_m, const PassArgs& p, const LastArgs& la, hipStream_t s)
 {
     return with_log_m(log_m, [&](auto lc) -> hipError_t {
         constexpr int LOG_M = decltype(lc)::value;
-        if ((p.frames - p.frame0) << LOG_M <= SMALL_VALUES)
-            return launch_tiles<LOG_M, 256>(p, la, s);
-        return launch_tiles<LOG_M, 512>(p, la, s);
+        const uint64_t values = (p.frames - p.frame0) << LOG_M;
+        if constexpr (LOG_M <= 18) {
+            if (values <= TINY_VALUES)
+                return launch_tiles<LOG_M, 128>(p, la, s);
+        }
+        if constexpr (LOG_M >= 16) {
+            if (values > SMALL_VALUES)
+                return launch_tiles<LOG_M, 512>(p, la, s);
+        }
+        return launch_tiles<LOG_M, 256>(p, la, s);
     });
 }
 
 }  // namespace
 
-bool multipass_supported(int log_m) { return log_m >= 16 && log_m <= 19; }
+bool multipass_supported(int log_m) { return log_m >= 15 && log_m <= 19; }
 
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m)
 {
@@ -490,6 +522,7 @@ int pass_tables(ostft_ctx* ctx, int log_m, bool noalloc, PassTables* t)
 {
     int rc = OSTFT_OK;
     const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
+    t->r1 = nullptr;
     if ((t->r0 = ctx_twiddles(ctx, MP_R0, MP_R0, &rc, noalloc)))
         t->r1 = ctx_twiddles(ctx, R1, R1, &rc, noalloc);
     for (int j = 0; rc == OSTFT_OK && j < log_m - MP_LOG_R0; ++j)
@@ -608,6 +641,29 @@ hipError_t multipass_static_scratch_init(int device)
         return e;
     static_ptr[device] = static_cast<float2*>(ptr);
     return hipSuccess;
+}
+
+// Window 2^16: the one kernel keeps a CU busy with a frame, so a request of few
+// frames leaves the GPU idle; up to 56 frames take the two passes, four or eight
+// workgroups a frame, with the same arithmetic (M = 32 x 32 x 32 either way).  One
+// kernel / two passes, power: 5 frames 23.5 / 15.7 us, 20 23.5 / 17.6, 36 23.8 / 20.8,
+// 52 24.1 / 23.1, 64 24.2 / 24.8, 80 24.3 / 29.8; complex half: 3 frames 28.6 / 15.8, 48
+// 28.5 / 24.7, 64 29.0 / 26.5, 96 29.0 / 32.5.
+constexpr uint64_t WIDE_IN_PASSES = 56;
+
+int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
+{
+    if (a.frames <= WIDE_IN_PASSES) {
+        bool room;  // in chunks of a small budget the passes would be the slower form
+        {
+            std::lock_guard<std::mutex> lk(ctx_scratch_mutex(ctx));
+            room = multipass_chunk_frames(ctx_scratch(ctx).budget, log_m) >= a.frames;
+        }
+        if (room)
+            return run_multipass(ctx, log_m, a, s);
+    }
+    const hipError_t e = launch_wide(a, 1, s);
+    return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "wide STFT launch");
 }
 
 int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)

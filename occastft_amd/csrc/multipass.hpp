@@ -1,4 +1,5 @@
-// multipass.hpp -- large-window path (complex transform sizes 2^16 .. 2^19).
+// multipass.hpp -- large-window path (complex transform sizes 2^16 .. 2^19, and
+// short requests of 2^15).
 #pragma once
 
 #include <mutex>
@@ -38,6 +39,8 @@ std::mutex& ctx_scratch_mutex(ostft_ctx* ctx);  // held while a call queues its 
 
 // Runs the two passes (the split epilogue inside the last).  Returns an OSTFT_* status.
 int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
+// Window 2^16: the two passes for a few frames, else the one kernel (bitwise the same).
+int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
 // The same through the fixed per-device scratch array (no allocation, no
 // event; the tables must be resident).  Calls that overlap on one GPU race.
 int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs& a, hipStream_t s);
@@ -48,6 +51,6 @@ hipError_t multipass_static_scratch_init(int device);
 // between the two passes at any time.
 uint64_t multipass_chunk_frames(uint64_t budget, int log_m);
 
-bool multipass_supported(int log_m);  // complex sizes 2^16 .. 2^19
+bool multipass_supported(int log_m);  // complex sizes 2^15 .. 2^19
 
 }  // namespace ostft

@@ -238,8 +238,8 @@ class Runner:
         return cur.value
 
     def scratch_budget(self, nbytes: int = 0) -> int:
-        """Scratch budget (bytes) of the two-pass path for windows 2^17..2^20;
-        0 leaves it.  Returns the budget in force."""
+        """Scratch budget (bytes) of the two-pass path (windows 2^17..2^20 and
+        short requests at 2^16); 0 leaves it.  Returns the budget in force."""
         cur = ctypes.c_uint64()
         rc = N.lib().ostft_scratch_budget(self._h, int(nbytes), ctypes.byref(cur))
         if rc != N.OK:
