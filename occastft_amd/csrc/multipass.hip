@@ -644,18 +644,25 @@ hipError_t multipass_static_scratch_init(int device)
 }
 
 // Window 2^16: the one kernel keeps a CU busy with a frame, so a request of few
-// frames leaves the GPU idle; up to 56 frames take the two passes, four or eight
+// frames leaves the GPU idle; up to 56 frames (64 of the complex layout, whose
+// stores take the one kernel longer) take the two passes, four or eight
 // workgroups a frame, with the same arithmetic (M = 32 x 32 x 32 either way).  One
 // kernel / two passes, power: 5 frames 23.5 / 15.7 us, 20 23.5 / 17.6, 36 23.8 / 20.8,
 // 52 24.1 / 23.1, 64 24.2 / 24.8, 80 24.3 / 29.8; complex half: 3 frames 28.6 / 15.8, 48
 // 28.5 / 24.7, 64 29.0 / 26.5, 96 29.0 / 32.5.
-constexpr uint64_t WIDE_IN_PASSES = 56;
+constexpr uint64_t WIDE_IN_PASSES = 56, WIDE_IN_PASSES_COMPLEX = 64;
 
 int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 {
-    if (a.frames <= WIDE_IN_PASSES) {
-        bool room;  // in chunks of a small budget the passes would be the slower form
-        {
+    if (a.frames <= (a.out_mode == OUT_HALF_COMPLEX ? WIDE_IN_PASSES_COMPLEX : WIDE_IN_PASSES)) {
+        // a captured call takes the one kernel, which needs no scratch: the graph
+        // then holds no address of a buffer that another call may grow
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        const hipError_t q = hipStreamIsCapturing(s, &cs);
+        if (q != hipSuccess)
+            (void)hipGetLastError();  // the launch below reads the last error
+        bool room = q == hipSuccess && cs == hipStreamCaptureStatusNone;
+        if (room) {  // in chunks of a small budget the passes would be the slower form
             std::lock_guard<std::mutex> lk(ctx_scratch_mutex(ctx));
             room = multipass_chunk_frames(ctx_scratch(ctx).budget, log_m) >= a.frames;
         }

@@ -31,7 +31,8 @@ def _signal(n, offset):
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("L,ov,offset", [(5, 0.0, 0), (65535, 0.5, 3), (1 << 16, 0.0, 0), (300_001, 0.33, 1),
                                          (16 << 16, 0.0, 1), (20 << 16, 0.0, 0), (21 << 16, 0.25, 2),
-                                         (55 << 16, 0.0, 0), (56 << 16, 0.0, 3)])
+                                         (55 << 16, 0.0, 0), (56 << 16, 0.0, 3),
+                                         (127 << 16, 0.0, 0), (128 << 16, 0.0, 0)])
 def test_passes_equal_the_one_kernel(runner, layout, L, ov, offset):
     import torch
 
@@ -59,6 +60,31 @@ def test_every_form_gives_the_same_frames(runner):
     (job,) = runner.run_batch_device([(x, p, None)])
     for got in (one[0], two[0], two[1], job):
         assert torch.equal(got[: want.numel()], want)
+
+
+def test_captured_call_takes_the_one_kernel():
+    """A context that has run only a long request at 2^16 holds neither the
+    scratch nor the tables of the two passes: a short one is captured all the
+    same, and its replays follow new inputs and eager work between."""
+    import torch
+
+    torch.zeros(1, device="cuda")
+    with ostft.Runner(0) as r:
+        p = ostft.parse_options("--hanning_window --power_return", 16, 0.5)
+        r.run_device(_signal(100 << 16, 0), p)
+        x = torch.zeros(5 << 16, device="cuda")
+        out = torch.zeros(ostft.geometry(p, x.numel())["out_floats"], device="cuda")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            r.run_device(x, p, out=out)
+        for rep in range(3):
+            x.normal_(generator=torch.Generator("cuda").manual_seed(rep))
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            got = out.clone()
+            assert torch.equal(got, r.run_device(x, p)), rep
 
 
 @pytest.mark.parametrize("exp,frames", [(17, 10), (18, 5), (19, 2)])
