@@ -208,9 +208,13 @@ typedef struct ostft_job {
  * request's result is bitwise identical to running it alone with
  * ostft_run_device.  All requests are validated before anything is launched;
  * a bad one fails the call (its index is in ostft_last_error).  Queued on
- * `hip_stream`, no wait.  Outputs must not overlap.  A batch of three or more
- * window sizes is refused (OSTFT_ERR_UNSUPPORTED) while the stream is being
- * captured: its records are rewritten by later batches. */
+ * `hip_stream`, no wait.  Outputs must not overlap.  While the stream is being
+ * captured, a batch of one or two window sizes (2^6..2^15) becomes part of the
+ * graph with request records of its own, which stay allocated until the context
+ * is destroyed (256 such batches and 64 MiB at most; further ones are captured
+ * as a launch per request), so its replays do not depend on later batches; the
+ * graph must not be replayed after ostft_destroy.  A batch of three or more
+ * window sizes is refused (OSTFT_ERR_UNSUPPORTED) under capture. */
 int ostft_run_batch_device(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, void* hip_stream);
 
 /* Floats each request's layout writes (ostft_geometry.out_floats), 0 for a

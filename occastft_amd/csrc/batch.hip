@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "batch.hpp"
+#include "capture.hpp"
 #include "multipass.hpp"
 #include "side_stream.hpp"
 
@@ -39,6 +40,9 @@ constexpr int LOG_M_MIN = 5, LOG_M_MAX = 14, NCLS = LOG_M_MAX - LOG_M_MIN + 1;
 constexpr size_t ALIGN = 256;
 // batches from so many tiles, and so many a request, use two streams (run_batch)
 constexpr uint64_t SIDE_TILES = 32768, SIDE_TILES_PER_REQUEST = 64;
+// captured batches keep so many blocks, and so many bytes of them, with the
+// context; beyond that a captured batch is a launch per request, which keeps nothing
+constexpr size_t HELD_BATCHES = 256, HELD_BYTES = (size_t)64 << 20;
 
 size_t align_up(size_t x) { return (x + ALIGN - 1) & ~(ALIGN - 1); }
 
@@ -53,7 +57,8 @@ static_assert(sizeof(BatchJob) % 8 == 0 && sizeof(BatchUpload) % 8 == 0, "copied
 
 // One descriptor block (claim counters, BatchJob records, tile table), the
 // pinned records it is filled from, and the event after the last launch that
-// reads it (both are reused only after it).
+// reads it (both are reused only after it).  A captured batch's block and
+// records are its own: every replay reads them.
 struct Slot {
     char* d = nullptr;
     size_t d_cap = 0;
@@ -68,6 +73,8 @@ struct Slot {
 struct BatchState {
     Slot slot[2];
     int next = 0;
+    std::vector<Slot> held;  // of captured batches
+    size_t held_bytes = 0;
     int cu_count = 0;
     int persistent[NCLS] = {};  // 1: persistent grid claiming tiles; 0: one workgroup per tile
     int per_cu[NCLS] = {};      // persistent workgroups per CU; 0: the occupancy limit
@@ -160,35 +167,87 @@ __global__ void __launch_bounds__(FILL_THREADS)
         tiles[at + i] = index;
 }
 
-hipError_t ensure_slot(Slot& sl, size_t d_bytes, size_t records)
+hipError_t ensure_block(Slot& sl, size_t d_bytes)
 {
-    if (sl.d_cap < d_bytes) {
-        if (sl.d)
-            (void)hipFree(sl.d);
+    if (sl.d_cap >= d_bytes)
+        return hipSuccess;
+    if (sl.d)
+        (void)hipFree(sl.d);
+    sl.d_cap = 0;
+    const hipError_t e = hipMalloc(&sl.d, d_bytes);
+    if (e == hipSuccess)
+        sl.d_cap = d_bytes;
+    else
         sl.d = nullptr;
-        sl.d_cap = 0;
-        const size_t cap = std::max<size_t>(align_up(d_bytes + d_bytes / 2), 64 * 1024);
-        const hipError_t e = hipMalloc(&sl.d, cap);
-        if (e != hipSuccess) {
-            sl.d = nullptr;
-            return e;
-        }
-        sl.d_cap = cap;
-    }
-    if (sl.h_cap < records) {
-        if (sl.h)
-            (void)hipHostFree(sl.h);
+    return e;
+}
+
+hipError_t ensure_records(Slot& sl, size_t records)
+{
+    if (sl.h_cap >= records)
+        return hipSuccess;
+    if (sl.h)
+        (void)hipHostFree(sl.h);
+    sl.h_cap = 0;
+    const hipError_t e = hipHostMalloc(&sl.h, records * sizeof(BatchUpload), hipHostMallocDefault);
+    if (e == hipSuccess)
+        sl.h_cap = records;
+    else
         sl.h = nullptr;
-        sl.h_cap = 0;
-        const size_t cap = std::max<size_t>(records + records / 2, 256);
-        const hipError_t e = hipHostMalloc(&sl.h, cap * sizeof(BatchUpload), hipHostMallocDefault);
-        if (e != hipSuccess) {
-            sl.h = nullptr;
-            return e;
-        }
-        sl.h_cap = cap;
+    return e;
+}
+
+void free_slot(Slot& sl)
+{
+    if (sl.d)
+        (void)hipFree(sl.d);
+    if (sl.h)
+        (void)hipHostFree(sl.h);
+    if (sl.done)
+        (void)hipEventDestroy(sl.done);
+    sl = Slot{};
+}
+
+// The next of the two blocks that batches take in turn, once the GPU is done with it.
+int next_slot(ostft_ctx* ctx, BatchState* st, size_t d_bytes, size_t records, Slot** out)
+{
+    Slot& sl = st->slot[st->next];
+    st->next ^= 1;
+    if (sl.used) {
+        const hipError_t e = hipEventSynchronize(sl.done);
+        if (e != hipSuccess)
+            return ctx_hip_fail(ctx, e, "batch slot wait");
     }
-    return hipSuccess;
+    hipError_t e = hipSuccess;
+    if (sl.d_cap < d_bytes)
+        e = ensure_block(sl, std::max<size_t>(align_up(d_bytes + d_bytes / 2), 64 * 1024));
+    if (e == hipSuccess && sl.h_cap < records)
+        e = ensure_records(sl, std::max<size_t>(records + records / 2, 256));
+    if (e != hipSuccess)
+        return ctx_hip_fail(ctx, e, "batch descriptor block");
+    *out = &sl;
+    return OSTFT_OK;
+}
+
+// A captured batch's own block; null beyond the bound or without memory for it.
+Slot* held_slot(BatchState* st, size_t d_bytes, size_t records)
+{
+    const size_t bytes = d_bytes + records * sizeof(BatchUpload);
+    if (st->held.size() >= HELD_BATCHES || st->held_bytes + bytes > HELD_BYTES)
+        return nullptr;
+    const AllocateInCapture allow(true);
+    Slot sl;
+    hipError_t e = ensure_block(sl, d_bytes);
+    if (e == hipSuccess)
+        e = ensure_records(sl, records);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        free_slot(sl);
+        return nullptr;
+    }
+    st->held_bytes += bytes;
+    st->held.push_back(sl);
+    return &st->held.back();
 }
 
 }  // namespace
@@ -256,43 +315,36 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
     for (int c = 0; c < NCLS; ++c)
         if (ntiles[c] >= 0x7fffffffull - 2ull * (uint64_t)st->cu_count * 64u)  // grid limit; claims overrun by <= 2/workgroup
             return ctx_fail(ctx, OSTFT_ERR_TOO_LARGE, "more than 2^31 tiles of one window size in a batch");
-    if (__builtin_popcount(mask) >= 3) {
-        // A captured batch replays from records that the next batch but one
-        // rewrites.  Batches of one or two window sizes may be captured by a caller
-        // who sees to that; with more it is refused.
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        const hipError_t e = hipStreamIsCapturing(s, &cs);
-        if (e != hipSuccess)
-            return ctx_hip_fail(ctx, e, "batch stream");
-        if (cs != hipStreamCaptureStatusNone)
-            return ctx_fail(ctx, OSTFT_ERR_UNSUPPORTED, "a batch of three or more window sizes cannot be captured");
+    const Capture capture = mask ? capture_of(s) : Capture{};
+    if (capture.on && __builtin_popcount(mask) >= 3)
+        return ctx_fail(ctx, OSTFT_ERR_UNSUPPORTED, "a batch of three or more window sizes cannot be captured");
+    // 3. descriptor block: claim counters, requests class by class, tile tables
+    //    class by class
+    size_t nreq = 0;
+    uint64_t total = 0, most = 0;
+    size_t first_job[NCLS] = {};
+    uint64_t first_tile[NCLS] = {};
+    for (int c = 0; c < NCLS; ++c) {
+        first_job[c] = nreq;
+        first_tile[c] = total;
+        nreq += members[c].size();
+        total += ntiles[c];
+    }
+    const size_t jobs_off = align_up(sizeof(uint32_t) * NCLS);
+    const size_t tiles_off = align_up(jobs_off + sizeof(BatchJob) * nreq);
+    const size_t d_bytes = tiles_off + sizeof(uint32_t) * total;
+    Slot* slot = nullptr;
+    std::vector<uint32_t> single;  // requests with a launch each, their arguments in it
+    if (capture.on) {
+        slot = held_slot(st, d_bytes, nreq);
+        for (int c = 0; !slot && c < NCLS; ++c)
+            single.insert(single.end(), members[c].begin(), members[c].end());
+        mask = slot ? mask : 0;
+    } else if (mask && (rc = next_slot(ctx, st, d_bytes, nreq, &slot)) != OSTFT_OK) {
+        return rc;
     }
     if (mask) {
-        // 3. descriptor block layout: claim counters, requests class by class,
-        //    tile tables class by class
-        size_t nreq = 0;
-        uint64_t total = 0, most = 0;
-        size_t first_job[NCLS] = {};
-        uint64_t first_tile[NCLS] = {};
-        for (int c = 0; c < NCLS; ++c) {
-            first_job[c] = nreq;
-            first_tile[c] = total;
-            nreq += members[c].size();
-            total += ntiles[c];
-        }
-        const size_t jobs_off = align_up(sizeof(uint32_t) * NCLS);
-        const size_t tiles_off = align_up(jobs_off + sizeof(BatchJob) * nreq);
-        const int si = st->next;
-        st->next ^= 1;
-        Slot& sl = st->slot[si];
-        if (sl.used) {
-            const hipError_t e = hipEventSynchronize(sl.done);
-            if (e != hipSuccess)
-                return ctx_hip_fail(ctx, e, "batch slot wait");
-        }
-        hipError_t e = ensure_slot(sl, tiles_off + sizeof(uint32_t) * total, nreq);
-        if (e != hipSuccess)
-            return ctx_hip_fail(ctx, e, "batch descriptor block");
+        Slot& sl = *slot;
         // 4. the requests' records
         for (int c = 0; c < NCLS; ++c) {
             uint64_t t = 0;
@@ -315,7 +367,7 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         const uint32_t parts = (uint32_t)std::min<uint64_t>(1 + most / (16 * FILL_THREADS), 256);
         hipLaunchKernelGGL(stft_batch_table_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj,
                            tj, counters);
-        e = hipGetLastError();
+        hipError_t e = hipGetLastError();
         // A large batch runs its classes on two streams in turn: the last tiles of
         // one class leave the GPU to the other stream's.  256 mixed requests
         // (47762 tiles of six classes): 470 -> 441 us (454 with each class on the
@@ -342,10 +394,18 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
             const hipError_t j = st->side.join(s);
             e = e == hipSuccess ? j : e;
         }
-        // also after a failed launch: what was queued may still read this slot
-        const hipError_t r = hipEventRecord(sl.done, s);
-        sl.used = sl.used || r == hipSuccess;
-        e = e == hipSuccess ? r : e;
+        if (!capture.on) {  // also after a failed launch: what was queued may still read this slot
+            const hipError_t r = hipEventRecord(sl.done, s);
+            sl.used = sl.used || r == hipSuccess;
+            e = e == hipSuccess ? r : e;
+        }
+        if (e != hipSuccess)
+            return ctx_hip_fail(ctx, e, "batch launch");
+    }
+    for (uint32_t i : single) {
+        FusedArgs& a = args[i];
+        a.tile_frames = (int32_t)fused_tile_frames((uint64_t)fused_variant_frames(lm[i], a.plan), 2ull << lm[i], a.hop);
+        const hipError_t e = launch_fused(lm[i], XF_FP32, a, 1, s);
         if (e != hipSuccess)
             return ctx_hip_fail(ctx, e, "batch launch");
     }
@@ -650,13 +710,10 @@ void batch_release(ostft_ctx* ctx)
     for (auto& sl : b->slot) {
         if (sl.used)
             (void)hipEventSynchronize(sl.done);
-        if (sl.d)
-            (void)hipFree(sl.d);
-        if (sl.h)
-            (void)hipHostFree(sl.h);
-        if (sl.done)
-            (void)hipEventDestroy(sl.done);
+        free_slot(sl);
     }
+    for (auto& sl : b->held)
+        free_slot(sl);
     b->side.destroy();
     delete b;
     b = nullptr;
