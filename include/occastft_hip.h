@@ -209,12 +209,13 @@ typedef struct ostft_job {
  * ostft_run_device.  All requests are validated before anything is launched;
  * a bad one fails the call (its index is in ostft_last_error).  Queued on
  * `hip_stream`, no wait.  Outputs must not overlap.  While the stream is being
- * captured, a batch of one or two window sizes (2^6..2^15) becomes part of the
- * graph with request records of its own, which stay allocated until the context
- * is destroyed (256 such batches and 64 MiB at most; further ones are captured
- * as a launch per request), so its replays do not depend on later batches; the
- * graph must not be replayed after ostft_destroy.  A batch of three or more
- * window sizes is refused (OSTFT_ERR_UNSUPPORTED) under capture. */
+ * captured, a batch becomes part of the graph with request records of its own,
+ * which stay allocated until the context is destroyed (256 such batches and 64
+ * MiB at most; further ones are captured as a launch per request), so its
+ * replays do not depend on later batches; the graph must not be replayed after
+ * ostft_destroy.  A batch of three or more window sizes (2^6..2^15) is refused
+ * (OSTFT_ERR_UNSUPPORTED) under capture unless ostft_batch_config turned
+ * use_graphs off. */
 int ostft_run_batch_device(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, void* hip_stream);
 
 /* Floats each request's layout writes (ostft_geometry.out_floats), 0 for a
@@ -226,9 +227,10 @@ int ostft_batch_out_floats(const ostft_job* jobs, uint32_t njobs, uint64_t* out_
  * selects the persistent form with that many workgroups per CU (clamped to
  * the occupancy limit; it also sets workgroup shape 0, the only one the
  * persistent kernel is built for), < 0 the one-workgroup-per-tile form (the
- * default), 0 leaves it (exp 0 too); use_graphs has no effect: launches are
- * direct, which is faster than replaying captured ones for every mix of window
- * sizes; *current receives the setting in force (0 for one workgroup per tile). */
+ * default), 0 leaves it (exp 0 too); use_graphs 1 (the default) refuses a batch
+ * of three or more window sizes on a stream that is being captured, 0 takes it,
+ * -1 leaves the setting (launches are direct either way); *current receives the
+ * launch form in force (0 for one workgroup per tile). */
 int ostft_batch_config(ostft_ctx* ctx, int32_t exp, int32_t blocks_per_cu, int32_t use_graphs,
                        int32_t* current);
 
@@ -298,7 +300,7 @@ typedef struct ostft_server_config {
     uint64_t arena_bytes;   /* device arena for admitted requests; 0: 1 GiB */
     uint32_t max_batch;     /* requests per batch; 0: 512 */
     uint32_t max_inflight;  /* batches on the GPU at once; 0: 3 */
-    int32_t use_graphs;     /* no effect (see ostft_batch_config) */
+    int32_t use_graphs;     /* no effect: a server's batches are never captured */
     int32_t autotune;       /* 1: autotune every batch window size (ostft_autotune_batch) at creation */
     const ostft_params* autotune_like; /* the requests to tune for (NULL: ostft_autotune_batch's default);
                                           read at creation only */

@@ -75,6 +75,7 @@ struct BatchState {
     int next = 0;
     std::vector<Slot> held;  // of captured batches
     size_t held_bytes = 0;
+    bool use_graphs = true;  // batch_config's; off: a batch of any number of sizes may be captured
     int cu_count = 0;
     int persistent[NCLS] = {};  // 1: persistent grid claiming tiles; 0: one workgroup per tile
     int per_cu[NCLS] = {};      // persistent workgroups per CU; 0: the occupancy limit
@@ -316,7 +317,7 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         if (ntiles[c] >= 0x7fffffffull - 2ull * (uint64_t)st->cu_count * 64u)  // grid limit; claims overrun by <= 2/workgroup
             return ctx_fail(ctx, OSTFT_ERR_TOO_LARGE, "more than 2^31 tiles of one window size in a batch");
     const Capture capture = mask ? capture_of(s) : Capture{};
-    if (capture.on && __builtin_popcount(mask) >= 3)
+    if (capture.on && st->use_graphs && __builtin_popcount(mask) >= 3)
         return ctx_fail(ctx, OSTFT_ERR_UNSUPPORTED, "a batch of three or more window sizes cannot be captured");
     // 3. descriptor block: claim counters, requests class by class, tile tables
     //    class by class
@@ -437,12 +438,14 @@ int class_of(ostft_ctx* ctx, int exp, int* c)
 
 }  // namespace
 
-int batch_config(ostft_ctx* ctx, int exp, int blocks_per_cu, int* current)
+int batch_config(ostft_ctx* ctx, int exp, int blocks_per_cu, int use_graphs, int* current)
 {
     BatchState* st = nullptr;
     int rc = state(ctx, &st);
     if (rc != OSTFT_OK)
         return rc;
+    if (use_graphs >= 0)
+        st->use_graphs = use_graphs != 0;
     if (exp == 0)
         return OSTFT_OK;
     int c = 0;

@@ -772,8 +772,7 @@ int ostft_batch_config(ostft_ctx* ctx, int32_t exp, int32_t blocks_per_cu, int32
     if (!dg.ok)
         return fail(ctx, OSTFT_ERR_NO_DEVICE, "hipSetDevice failed");
     std::lock_guard<std::mutex> lk(ctx->batch_mu);
-    (void)use_graphs;  // launches are direct either way
-    return ostft::batch_config(ctx, exp, blocks_per_cu, current);
+    return ostft::batch_config(ctx, exp, blocks_per_cu, use_graphs, current);
 }
 
 int ostft_engine_variant(ostft_ctx* ctx, int32_t exp, int32_t shape, int32_t plan, int32_t* cur_shape,

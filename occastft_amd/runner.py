@@ -229,8 +229,10 @@ class Runner:
 
     def batch_config(self, exp: int = 0, blocks_per_cu: int = 0, use_graphs: int = -1) -> int:
         """blocks_per_cu > 0: persistent form with that many workgroups per CU;
-        < 0: one workgroup per tile; 0: unchanged.  Returns the setting in
-        force (0 = one workgroup per tile)."""
+        < 0: one workgroup per tile; 0: unchanged.  use_graphs: 0 lets a batch
+        of three or more window sizes be captured into a graph, 1 (the default
+        of a context) refuses it, -1 leaves that; launches are direct either
+        way.  Returns the launch form in force (0 = one workgroup per tile)."""
         cur = ctypes.c_int32()
         rc = N.lib().ostft_batch_config(self._h, int(exp), int(blocks_per_cu), int(use_graphs), ctypes.byref(cur))
         if rc != N.OK:
@@ -296,7 +298,7 @@ class Server:
 
     ``submit`` queues a request and returns a ticket; ``wait`` returns the
     result array.  Input and output arrays are kept referenced here until the
-    request is waited for."""
+    request is waited for.  ``use_graphs`` has no effect."""
 
     def __init__(self, device: int = 0, arena_bytes: int = 0, max_batch: int = 0, max_inflight: int = 0,
                  use_graphs: bool = True, autotune: bool = False, autotune_like: N.Params | None = None,
