@@ -82,7 +82,7 @@ struct BatchState {
     int shape[NCLS] = {};       // workgroup shape (engine variant / 4); persistent needs 0
     int plan_override[NCLS];    // >= 0: radix plan for this class instead of the context's (autotuning)
     int variant[NCLS] = {};     // engine variant of each class in the current batch
-    SideStream side;
+    SideStreams sides;
     BatchClassInfo info[NCLS][FUSED_VARIANTS] = {};
     bool info_ok[NCLS][FUSED_VARIANTS] = {};
 
@@ -375,24 +375,25 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         // stream with fewer tiles so far); the fork and join cost the host 20 us, more than a smaller batch
         // gains (256 requests of 12000 tiles 220 -> 258 us).
         const bool two = total >= SIDE_TILES && total >= SIDE_TILES_PER_REQUEST * nreq && __builtin_popcount(mask) > 1;
-        if (e == hipSuccess && two)
-            e = st->side.fork(s);
-        const bool forked = e == hipSuccess && two;
+        SideStream* const other = two ? &st->sides.of(capture) : nullptr;
+        if (e == hipSuccess && other)
+            e = other->fork(s);
+        const bool forked = e == hipSuccess && other;
         int turn = 0;
         for (int c = 0; e == hipSuccess && c < NCLS; ++c) {
             if (!(mask >> c & 1u))
                 continue;
-            const bool side = two && (turn++ & 1);
+            const bool side = other && (turn++ & 1);
             BatchClassArgs a;
             a.jobs = bj + first_job[c];
             a.tile_job = tj + first_tile[c];
             a.counter = counters + c;
             a.ntiles = (uint32_t)ntiles[c];
             e = launch_batch(c + LOG_M_MIN, st->variant[c], a, class_grid(st, c, ntiles[c]), st->persistent[c] != 0,
-                             side ? st->side.stream : s);
+                             side ? other->stream : s);
         }
         if (forked) {  // also after a failed launch: what follows on s comes after the side stream's work
-            const hipError_t j = st->side.join(s);
+            const hipError_t j = other->join(s);
             e = e == hipSuccess ? j : e;
         }
         if (!capture.on) {  // also after a failed launch: what was queued may still read this slot
@@ -717,7 +718,7 @@ void batch_release(ostft_ctx* ctx)
     }
     for (auto& sl : b->held)
         free_slot(sl);
-    b->side.destroy();
+    b->sides.destroy();
     delete b;
     b = nullptr;
 }

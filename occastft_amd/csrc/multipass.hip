@@ -104,7 +104,7 @@ void Scratch::destroy()
     if (done)
         (void)hipEventDestroy(done);
     done = nullptr;
-    side.destroy();
+    sides.destroy();
     used = false;
 }
 
@@ -573,9 +573,9 @@ uint64_t chunk_frames(const Chunks& c, uint64_t left, uint64_t cap)
 }
 
 // Both passes over the request's frames, chunk by chunk through `buf` (`cap`
-// frames; two such buffers with `sc`, whose side stream takes every other chunk).
+// frames; two such buffers with `other`, which takes every other chunk).
 int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& t, float2* buf, uint64_t cap,
-               const Chunks& c, hipStream_t s, Scratch* sc = nullptr)
+               const Chunks& c, hipStream_t s, SideStream* other = nullptr)
 {
     PassArgs p;
     p.sig = a.in;
@@ -594,20 +594,20 @@ int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& 
     la.out_mode = a.out_mode;
     la.dc = a.dc;
 
-    hipError_t e = sc ? sc->side.fork(s) : hipSuccess;
+    hipError_t e = other ? other->fork(s) : hipSuccess;
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass side stream");
     uint32_t i = 0;
     for (uint64_t f0 = 0; e == hipSuccess && f0 < a.frames; f0 = p.frames, ++i) {
-        const bool side = sc && (i & 1u);
+        const bool side = other && (i & 1u);
         p.dst = buf + (side ? cap << log_m : 0);
         la.src = p.dst;
         p.frame0 = la.frame0 = f0;
         p.frames = la.frames = f0 + chunk_frames(c, a.frames - f0, cap);
-        e = launch_passes(log_m, p, la, side ? sc->side.stream : s);
+        e = launch_passes(log_m, p, la, side ? other->stream : s);
     }
-    if (sc) {  // also after a failed launch: what follows on s comes after the side stream's work
-        const hipError_t j = sc->side.join(s);
+    if (other) {  // also after a failed launch: what follows on s comes after the side stream's work
+        const hipError_t j = other->join(s);
         e = e == hipSuccess ? j : e;
     }
     return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "multi-pass launch");
@@ -694,7 +694,7 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     PassTables t;
     int rc = pass_tables(ctx, log_m, false, &t);
     if (rc == OSTFT_OK)
-        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, c, s, c.two ? &sc : nullptr);
+        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, c, s, c.two ? &sc.sides.of(capture_of(s)) : nullptr);
     // also after a failed launch: what was queued may still use the scratch
     e = sc.handoff(s);
     if (rc != OSTFT_OK)

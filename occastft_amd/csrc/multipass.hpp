@@ -20,7 +20,7 @@ struct Scratch {
     uint64_t cap = 0;                      // complex elements
     uint64_t budget = (uint64_t)1 << 30;  // bytes it may take
     hipEvent_t done = nullptr;             // recorded after the last call's launches
-    SideStream side;                       // every other chunk of a long request runs here
+    SideStreams sides;                     // every other chunk of a long request runs on one of these
     hipStream_t last = nullptr;            // the stream of that call
     bool used = false;
     hipError_t ensure(uint64_t n);

@@ -5,6 +5,11 @@
 
 #include <hip/hip_runtime.h>
 
+#include <memory>
+#include <vector>
+
+#include "capture.hpp"
+
 namespace ostft {
 
 struct SideStream {
@@ -41,6 +46,43 @@ struct SideStream {
         if (stream)
             (void)hipStreamDestroy(stream);
         stream = nullptr;
+    }
+};
+
+// The side streams of one kind of launches (under its lock).  A stream forked
+// from a capturing one belongs to that capture until it ends, and another call
+// could not fork it: ordinary calls have a side stream of their own, and each
+// capture under way has one, which a later capture takes over.
+class SideStreams {
+    struct Captured {
+        SideStream side;
+        unsigned long long id;
+    };
+    SideStream own;
+    std::vector<std::unique_ptr<Captured>> captured;
+
+public:
+    SideStream& of(const Capture& c)
+    {
+        if (!c.on)
+            return own;
+        for (auto& k : captured)
+            if (k->id == c.id)
+                return k->side;
+        for (auto& k : captured)
+            if (!k->side.stream || !capture_of(k->side.stream).on) {
+                k->id = c.id;
+                return k->side;
+            }
+        captured.emplace_back(new Captured{SideStream{}, c.id});
+        return captured.back()->side;
+    }
+    void destroy()
+    {
+        own.destroy();
+        for (auto& k : captured)
+            k->side.destroy();
+        captured.clear();
     }
 };
 
