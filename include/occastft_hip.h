@@ -147,6 +147,13 @@ void ostft_destroy(ostft_ctx* ctx);
  * FP64-generated twiddle tables synchronously.  Windows 2^17..2^20 pass
  * through the context's scratch buffer: a call on another stream than the
  * previous such call first makes its stream wait for that call's launches.
+ * Under stream capture (with the tables resident) such a call, and a short one
+ * at 2^16, takes a buffer of its own, which stays allocated until the context is
+ * destroyed; the captured buffers of a context fit its scratch budget
+ * (ostft_scratch_budget).  Beyond it a window of 2^16 needs none, and a larger
+ * one captures the context's scratch buffer: that graph's replays must then be
+ * ordered with the context's other calls of these windows.  No graph may be
+ * replayed after ostft_destroy.
  * Replaces the device part of Runner::ActivateSTFT. */
 int ostft_run_device(ostft_ctx* ctx, const ostft_params* params, const float* d_in,
                      uint64_t full_size, float* d_out, uint64_t out_cap, void* hip_stream);
@@ -277,7 +284,8 @@ int ostft_autotune_batch(ostft_ctx* ctx, int32_t exp, uint64_t samples, const os
  * frames at 2^16 where the budget holds them), in bytes: its
  * frames go through both passes in chunks, and the intermediate spectra of the
  * chunks in work fit the budget (one frame always does).  bytes = 0 leaves
- * it; a budget below the scratch already held frees that scratch.  *current
+ * it; a budget below the scratch already held frees that scratch (what a
+ * captured graph uses stays).  *current
  * (may be NULL) receives the budget in force.  Default 1 GiB.  No counterpart in the
  * reference, whose runners hold whole-signal intermediate buffers. */
 int ostft_scratch_budget(ostft_ctx* ctx, uint64_t bytes, uint64_t* current);

@@ -353,6 +353,11 @@ float2* ctx_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noa
 {
     return get_twiddles(ctx, m, count, rc, noalloc);
 }
+bool ctx_has_twiddles(ostft_ctx* ctx, int64_t m, int64_t count)
+{
+    std::lock_guard<std::mutex> lk(ctx->mu);
+    return ctx->twiddles.count({m, count}) != 0;
+}
 Scratch& ctx_scratch(ostft_ctx* ctx) { return ctx->scratch; }
 std::mutex& ctx_scratch_mutex(ostft_ctx* ctx) { return ctx->scratch_mu; }
 BatchState*& ctx_batch(ostft_ctx* ctx) { return ctx->batch; }

@@ -85,9 +85,31 @@ hipError_t Scratch::handoff(hipStream_t s)
     return e;
 }
 
+float2* Scratch::hold(const Capture& c, hipStream_t s, uint64_t n)
+{
+    for (const Held& h : held)
+        if (h.capture == c.id && h.stream == s && h.cap >= n)
+            return h.a;
+    const uint64_t bytes = sizeof(float2) * n;
+    if (bytes > budget || held_bytes > budget - bytes)
+        return nullptr;
+    Held h{c.id, s, nullptr, n};
+    const AllocateInCapture allow(true);
+    if (hipMalloc(&h.a, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    held.push_back(h);
+    held_bytes += bytes;
+    return h.a;
+}
+
 void Scratch::release()
 {
-    if (a) {
+    if (a && in_graph) {
+        held.push_back(Held{0, nullptr, a, 0});  // for destroy(); serves no further call
+        held_bytes += sizeof(float2) * cap;
+    } else if (a) {
         // the last call's launches (on whatever stream) must be done with it;
         // other streams and contexts on the device are not waited for
         if (used && done)
@@ -96,11 +118,16 @@ void Scratch::release()
     }
     a = nullptr;
     cap = 0;
+    in_graph = false;
 }
 
 void Scratch::destroy()
 {
     release();
+    for (const Held& h : held)
+        (void)hipFree(h.a);
+    held.clear();
+    held_bytes = 0;
     if (done)
         (void)hipEventDestroy(done);
     done = nullptr;
@@ -530,6 +557,15 @@ int pass_tables(ostft_ctx* ctx, int log_m, bool noalloc, PassTables* t)
     return rc;
 }
 
+bool tables_resident(ostft_ctx* ctx, int log_m)
+{
+    const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
+    bool all = ctx_has_twiddles(ctx, MP_R0, MP_R0) && ctx_has_twiddles(ctx, R1, R1);
+    for (int j = 0; all && j < log_m - MP_LOG_R0; ++j)
+        all = ctx_has_twiddles(ctx, (int64_t)1 << (log_m - j), MP_R0);
+    return all;
+}
+
 // Frames go through both passes a chunk at a time, so that the last pass reads
 // scratch that is still in the 256 MB memory-side cache.  One chunk at a time:
 // 768 workgroups (96 MiB of scratch), what is left over joins the last chunk or
@@ -655,16 +691,16 @@ constexpr uint64_t WIDE_IN_PASSES = 56, WIDE_IN_PASSES_COMPLEX = 64;
 int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 {
     if (a.frames <= (a.out_mode == OUT_HALF_COMPLEX ? WIDE_IN_PASSES_COMPLEX : WIDE_IN_PASSES)) {
-        // a captured call takes the one kernel, which needs no scratch: the graph
-        // then holds no address of a buffer that another call may grow
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        const hipError_t q = hipStreamIsCapturing(s, &cs);
-        if (q != hipSuccess)
-            (void)hipGetLastError();  // the launch below reads the last error
-        bool room = q == hipSuccess && cs == hipStreamCaptureStatusNone;
-        if (room) {  // in chunks of a small budget the passes would be the slower form
+        const Capture capture = capture_of(s);
+        bool room;
+        {  // in chunks of a small budget the passes would be the slower form
             std::lock_guard<std::mutex> lk(ctx_scratch_mutex(ctx));
-            room = multipass_chunk_frames(ctx_scratch(ctx).budget, log_m) >= a.frames;
+            Scratch& sc = ctx_scratch(ctx);
+            room = multipass_chunk_frames(sc.budget, log_m) >= a.frames;
+            // a captured call takes the passes with a buffer of its own, and tables
+            // that are there (none can be built under capture)
+            if (room && capture.on)
+                room = tables_resident(ctx, log_m) && sc.hold(capture, s, a.frames << log_m);
         }
         if (room)
             return run_multipass(ctx, log_m, a, s);
@@ -685,18 +721,29 @@ int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
     const uint64_t room = multipass_chunk_frames(sc.budget, log_m);
     const Chunks c = chunks_of(a.frames, room, log_m, a.out_mode);
     const uint64_t cap = std::min(room, chunk_most(c, a.frames));
-    hipError_t e = sc.ensure((c.two ? 2 : 1) * cap * M);
-    if (e != hipSuccess)
-        return ctx_hip_fail(ctx, e, "multi-pass scratch allocation");
-    e = sc.acquire(s);
+    const uint64_t need = (c.two ? 2 : 1) * cap * M;
+    const Capture capture = capture_of(s);
+    float2* buf = capture.on ? sc.hold(capture, s, need) : nullptr;
+    hipError_t e = hipSuccess;
+    if (!buf) {
+        const AllocateInCapture allow(capture.on);
+        e = sc.ensure(need);
+        if (e != hipSuccess)
+            return ctx_hip_fail(ctx, e, "multi-pass scratch allocation");
+        buf = sc.a;
+        sc.in_graph |= capture.on;
+    }
+    if (!capture.on)  // a graph's launches are ordered by who replays it
+        e = sc.acquire(s);
     if (e != hipSuccess)
         return ctx_hip_fail(ctx, e, "multi-pass scratch ordering");
     PassTables t;
     int rc = pass_tables(ctx, log_m, false, &t);
     if (rc == OSTFT_OK)
-        rc = run_chunks(ctx, log_m, a, t, sc.a, cap, c, s, c.two ? &sc.sides.of(capture_of(s)) : nullptr);
+        rc = run_chunks(ctx, log_m, a, t, buf, cap, c, s, c.two ? &sc.sides.of(capture) : nullptr);
     // also after a failed launch: what was queued may still use the scratch
-    e = sc.handoff(s);
+    if (!capture.on)
+        e = sc.handoff(s);
     if (rc != OSTFT_OK)
         return rc;
     return e == hipSuccess ? OSTFT_OK : ctx_hip_fail(ctx, e, "multi-pass scratch event");

@@ -3,7 +3,9 @@
 #pragma once
 
 #include <mutex>
+#include <vector>
 
+#include "capture.hpp"
 #include "engine.hpp"
 #include "side_stream.hpp"
 
@@ -14,26 +16,39 @@ namespace ostft {
 // The complex buffer between the two passes, owned by a context, grown on
 // demand up to one chunk of frames.  Calls on different streams take turns:
 // each call's launches wait for the previous call's (an event recorded on
-// its stream) when the stream changes.
+// its stream) when the stream changes.  Captured calls have buffers of their own,
+// together up to the budget; beyond that a graph uses this one.  What a graph
+// uses is not freed before the context goes.
 struct Scratch {
+    struct Held {
+        unsigned long long capture;  // the calls of this capture on this stream
+        hipStream_t stream;
+        float2* a;
+        uint64_t cap;
+    };
     float2* a = nullptr;
     uint64_t cap = 0;                      // complex elements
+    bool in_graph = false;                 // a graph uses `a`
+    std::vector<Held> held;
+    uint64_t held_bytes = 0;
     uint64_t budget = (uint64_t)1 << 30;  // bytes it may take
     hipEvent_t done = nullptr;             // recorded after the last call's launches
     SideStreams sides;                     // every other chunk of a long request runs on one of these
     hipStream_t last = nullptr;            // the stream of that call
     bool used = false;
     hipError_t ensure(uint64_t n);
+    float2* hold(const Capture& c, hipStream_t s, uint64_t n);  // a captured call's buffer, or null
     hipError_t acquire(hipStream_t s);  // order stream s after the previous user
     hipError_t handoff(hipStream_t s);  // record the end of this call's launches
     void release();                     // frees the buffer (after the last user's launches)
-    void destroy();                     // release + the event
+    void destroy();                     // everything (no graph uses it any more)
 };
 
 // accessors into the context (defined in capi.hip)
 // W_m^j, j < count; with `noalloc` only a table already resident (else null
 // and OSTFT_ERR_NOT_PREPARED in *rc)
 float2* ctx_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc = false);
+bool ctx_has_twiddles(ostft_ctx* ctx, int64_t m, int64_t count);  // that table is resident
 Scratch& ctx_scratch(ostft_ctx* ctx);
 std::mutex& ctx_scratch_mutex(ostft_ctx* ctx);  // held while a call queues its scratch launches
 
