@@ -172,7 +172,10 @@ int ostft_run_device(ostft_ctx* ctx, const ostft_params* params, const float* d_
  *     event.  Every call on a GPU shares that array and it keeps the last
  *     call's contents (each call overwrites what it reads first): calls that
  *     overlap in time on one GPU race; keep them on one stream or ordered.
- * Windows up to 2^16 use no scratch here. */
+ * Windows up to 2^15 use no scratch.  A request of few frames at 2^16 uses the
+ * context's own scratch as ostft_run_device does, ordered across streams by an
+ * event, where earlier calls have made it large enough; else, and under capture,
+ * none. */
 int ostft_run_device_noalloc(ostft_ctx* ctx, const ostft_params* params, const float* d_in,
                              uint64_t full_size, float* d_out, uint64_t out_cap, void* hip_stream);
 

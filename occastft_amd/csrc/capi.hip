@@ -702,10 +702,8 @@ int ostft_run_device_noalloc(ostft_ctx* ctx, const ostft_params* params, const f
         hipError_t e = ostft::launch_fused(log_m, transform_of(params), a, 1, s);
         return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "fused STFT launch");
     }
-    if (ostft::wide_supported(log_m)) {
-        const hipError_t e = ostft::launch_wide(a, 1, s);
-        return e == hipSuccess ? OSTFT_OK : hip_fail(ctx, e, "wide STFT launch");
-    }
+    if (ostft::wide_supported(log_m))
+        return ostft::run_wide_noalloc(ctx, log_m, a, s);
     return ostft::run_multipass_static(ctx, ctx->device, log_m, a, s);
 }
 

@@ -52,10 +52,14 @@ bool ctx_has_twiddles(ostft_ctx* ctx, int64_t m, int64_t count);  // that table 
 Scratch& ctx_scratch(ostft_ctx* ctx);
 std::mutex& ctx_scratch_mutex(ostft_ctx* ctx);  // held while a call queues its scratch launches
 
-// Runs the two passes (the split epilogue inside the last).  Returns an OSTFT_* status.
-int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
+// Runs the two passes (the split epilogue inside the last).  Returns an OSTFT_*
+// status; with `noalloc`, OSTFT_ERR_NOT_PREPARED (and no message) where the
+// scratch that is there does not hold the request, or s is being captured.
+int run_multipass(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s, bool noalloc = false);
 // Window 2^16: the two passes for a few frames, else the one kernel (bitwise the same).
 int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
+// The same without allocations: the passes where scratch and tables are there.
+int run_wide_noalloc(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s);
 // The same through the fixed per-device scratch array (no allocation, no
 // event; the tables must be resident).  Calls that overlap on one GPU race.
 int run_multipass_static(ostft_ctx* ctx, int device, int log_m, const FusedArgs& a, hipStream_t s);
