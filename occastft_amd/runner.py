@@ -201,6 +201,8 @@ class Runner:
         for x, p, _ in jobs:
             if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
                 raise ValueError("inputs must be contiguous float32 tensors on the GPU")
+            if not isinstance(p, N.Params):
+                raise TypeError(f"params must be Params, not {type(p).__name__}")
             ptrs.append(x.data_ptr())
             sizes.append(x.numel())
             params.append(bytes(p))
