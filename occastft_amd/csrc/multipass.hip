@@ -393,6 +393,7 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
         constexpr bool COMB = decltype(comb_c)::value;
         constexpr bool CUT = decltype(cut_c)::value;  // HALF_COMPLEX: the frame that out_limit cuts short
         constexpr bool HALF = MODE == OUT_POWER || MODE == OUT_HALF_SPECTRUM;
+        static_assert(COMB || !HALF, "the layouts of N/2+1 values are of the full FFT");
         constexpr bool CPLX = MODE == OUT_HALF_COMPLEX || MODE == OUT_HALF_SPECTRUM;
         constexpr uint32_t B = CPLX ? 8 : 4;      // bytes of an output value
         constexpr uint32_t W = HALF ? M + 1 : N;  // values of a frame
@@ -418,10 +419,7 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
             const bool first = I == 0 && k0 && t == 0;  // bin 0 has no mirror below N
             put(lo, O, bp.lo, false);
             if constexpr (HALF) {
-                if (COMB || first)
-                    put(hi, M - Ns * T - O, bp.hi, !first);
-                else
-                    put(hi, M - Ns * T - O, bp.lo, true);
+                put(hi, M - Ns * T - O, bp.hi, !first);
             } else {
                 put(lo, M + O, bp.hi, false);
                 if (!first) {
@@ -568,8 +566,8 @@ bool tables_resident(ostft_ctx* ctx, int log_m)
 
 // Frames go through both passes a chunk at a time, so that the last pass reads
 // scratch that is still in the 256 MB memory-side cache.  One chunk at a time:
-// 768 workgroups (96 MiB of scratch), what is left over joins the last chunk or
-// makes one of at least half the size.  Requests of more than 2048 workgroups a
+// 768 workgroups (96 MiB of scratch); what is left over joins the last chunk, of 1152
+// (144 MiB) at most, or makes one of at least half the size.  Requests of more than 2048 workgroups a
 // pass run two chunks of 512 (one round of the GPU) at a time, every other one on
 // a side stream: the last workgroups of one chunk's launch leave the GPU to the
 // other chunk's, and one's loads meet the other's transforms.
