@@ -38,8 +38,21 @@ namespace {
 
 constexpr int LOG_M_MIN = 5, LOG_M_MAX = 14, NCLS = LOG_M_MAX - LOG_M_MIN + 1;
 constexpr size_t ALIGN = 256;
-// batches from so many tiles, and so many a request, use two streams (run_batch)
-constexpr uint64_t SIDE_TILES = 32768, SIDE_TILES_PER_REQUEST = 64;
+// Batches of so many window sizes and tiles, and so many tiles a request, use two
+// streams: the last tiles of one class leave the GPU to the other stream's.
+// One / two streams, requests of ten to sixty million samples in all, power.
+//   Sizes (calls from C, in a row; each waited for), 60 requests, 31000 tiles, 50%:
+//   two 264 / 265 and 274 / 293 us, three 284 / 278 and 293 / 304, four 298 / 290
+//   and 307 / 313, five 293 / 282 and 303 / 305; 256 requests, 33000 tiles, 60%: five
+//   310 / 295 and 326 / 325, six 326 / 309 and 357 / 340, eight 343 / 307 and 374 / 339.
+//   Tiles a request: while the host, at 0.9 us a request from Python, is the slower
+//   side, the fork and join cost it 60-100 us.  Six sizes, 60%, 400 requests of 91
+//   tiles 393 / 475, 111 459 / 486, 131 528 / 514, 182 698 / 679; 1024 of 90 927 / 1075,
+//   110 1099 / 1118, 130 1278 / 1261.
+//   Tiles: the same for few requests, 64 of 101 tiles 106 / 131; 256 of 111 301 / 327,
+//   of 132 364 / 343 (from C two streams win from 5000 tiles on).
+constexpr int SIDE_SIZES = 5;
+constexpr uint64_t SIDE_TILES = 32768, SIDE_TILES_PER_REQUEST = 128;
 // captured batches keep so many blocks, and so many bytes of them, with the
 // context; beyond that a captured batch is a launch per request, which keeps nothing
 constexpr size_t HELD_BATCHES = 256, HELD_BYTES = (size_t)64 << 20;
@@ -369,12 +382,11 @@ int run_batch(ostft_ctx* ctx, const ostft_job* jobs, uint32_t njobs, hipStream_t
         hipLaunchKernelGGL(stft_batch_table_kernel, dim3((uint32_t)nreq, parts), dim3(FILL_THREADS), 0, s, sl.h, bj,
                            tj, counters);
         hipError_t e = hipGetLastError();
-        // A large batch runs its classes on two streams in turn: the last tiles of
-        // one class leave the GPU to the other stream's.  256 mixed requests
+        // A large batch runs its classes on two streams in turn.  256 mixed requests
         // (47762 tiles of six classes): 470 -> 441 us (454 with each class on the
-        // stream with fewer tiles so far); the fork and join cost the host 20 us, more than a smaller batch
-        // gains (256 requests of 12000 tiles 220 -> 258 us).
-        const bool two = total >= SIDE_TILES && total >= SIDE_TILES_PER_REQUEST * nreq && __builtin_popcount(mask) > 1;
+        // stream with fewer tiles so far)
+        const bool two = total >= SIDE_TILES && total >= SIDE_TILES_PER_REQUEST * nreq &&
+                         __builtin_popcount(mask) >= SIDE_SIZES;
         SideStream* const other = two ? &st->sides.of(capture) : nullptr;
         if (e == hipSuccess && other)
             e = other->fork(s);

@@ -1,5 +1,5 @@
-"""Large batches run their window sizes on two streams (from 32768 tiles, and 64
-a request): every request bitwise as run alone, run three times in a row
+"""Large batches run their window sizes on two streams (from five sizes, 32768
+tiles, and 128 a request): every request bitwise as run alone, run three times in a row
 (both descriptor blocks, and one again) and followed, with no wait, by a batch
 that overwrites the inputs; and inside a graph capture, with a large batch on
 another stream of the same context meanwhile."""
@@ -8,8 +8,8 @@ import pytest
 import occastft_amd as ostft
 
 pytestmark = pytest.mark.gpu
-# a tile of 256 threads is 32, 8, 2 or 1 frames, at 75% overlap always 2048 samples apart
-EXPS = (8, 10, 12, 13)
+# a tile of 256 threads is 32, 16, 8, 4, 2 or 1 frames, at 75% overlap always 2048 samples apart
+EXPS = (8, 9, 10, 11, 12, 13)
 TILE_HOP = 2048
 
 
@@ -72,7 +72,8 @@ def test_captured_beside_another_streams_batch(runner):
     another stream forks meanwhile; the next capture takes it over."""
     import torch
 
-    captured, eager = _batch((8, 12) * 2, 2), _batch((10, 13) * 2, 3)
+    captured, eager = _batch(EXPS, 2), _batch(EXPS[::-1] * 2, 3)
+    runner.batch_config(use_graphs=0)  # a batch of many sizes may be captured
     want = [runner.run_device(x, p).clone() for x, p, _ in eager]
     for jobs in (captured, eager):
         runner.run_batch_device(jobs)
@@ -98,3 +99,4 @@ def test_captured_beside_another_streams_batch(runner):
         for x, p, out in captured:
             assert torch.equal(out, runner.run_device(x, p)), (rep, p.exp)
         assert all(int(out.count_nonzero()) == 0 for _, _, out in eager)
+    runner.batch_config(use_graphs=1)
