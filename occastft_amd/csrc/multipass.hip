@@ -567,13 +567,15 @@ bool tables_resident(ostft_ctx* ctx, int log_m)
 // Frames go through both passes a chunk at a time, so that the last pass reads
 // scratch that is still in the 256 MB memory-side cache.  One chunk at a time:
 // 768 workgroups (96 MiB of scratch); what is left over joins the last chunk, of 1152
-// (144 MiB) at most, or makes one of at least half the size.  Requests of more than 2048 workgroups a
-// pass run two chunks of 512 (one round of the GPU) at a time, every other one on
-// a side stream: the last workgroups of one chunk's launch leave the GPU to the
-// other chunk's, and one's loads meet the other's transforms.
-// One / two at a time, overlap 0.5, power: 2^17, 1400 workgroups 144 / 143 us, 2048
-// 209 / 202, 3000 294 / 271; 2^20 153 / 148, 224 / 216, 318 / 287 (below 1024 the fork
-// and join of the streams cost 10-20 us more than they give).  Scratch of one
+// (144 MiB) at most, or makes one of at least half the size.  Requests of more than
+// 2304 workgroups a pass run two chunks of 512 (one round of the GPU) at a time,
+// every other one on a side stream: the last workgroups of one chunk's launch leave
+// the GPU to the other chunk's, and one's loads meet the other's transforms.  The
+// fork and join of the streams cost 10-20 us.  One / two at a time, calls in a row
+// and each waited for: power, 75%, 2^17, 2080 workgroups 196 / 204 and 205 / 224 us,
+// 2400 224 / 217 and 233 / 237, 3200 300 / 289 and 316 / 310; 2^20, 2080 209 / 206 and
+// 218 / 225, 2500 242 / 233 and 252 / 252, 4096 396 / 365 and 413 / 387; default layout,
+// overlap 0, 2^17, 2200 250 / 253 and 260 / 272, 2500 285 / 269 and 294 / 288.  Scratch of one
 // chunk at a time of 64 / 96 / 128 / 256 / 1024 MiB, 2^26 samples, 75%, default
 // layout: 2^17 894 / 848 / 866 / 997 / 892 us; two at a time of 48 / 64 / 80 / 96 MiB each:
 // 805 / 773 / 863 / 890.
@@ -587,8 +589,12 @@ Chunks chunks_of(uint64_t frames, uint64_t room, int log_m, int out_mode)
     // the complex layout writes 16 bytes a value, which at 2^19 and 2^20 push the
     // second chunk's scratch out of the cache: 577 / 600 and 625 / 673 us (2^18 589 / 576)
     const bool wide = out_mode == OUT_HALF_COMPLEX && log_m >= 18;
+    // and the layouts of 8 bytes a value at 2^20 gain from twice as many workgroups on:
+    // default, overlap 0.5, 2300 273 / 278, 4096 486 / 465; 75%, 2300 262 / 269, 2800
+    // 319 / 322, 4096 473 / 462; overlap 0, 2300 288 / 299, 4096 517 / 521, 8192 1023 / 1018
+    const uint64_t from = log_m == 19 && out_mode != OUT_POWER ? 4096 : 2304;
     Chunks c;
-    c.two = values > 2048 * tile && room >= 2 * ((512 * tile) >> log_m) && !wide;
+    c.two = values > from * tile && room >= 2 * ((512 * tile) >> log_m) && !wide;
     c.want = ((c.two ? 512 : 768) * tile) >> log_m;
     return c;
 }
