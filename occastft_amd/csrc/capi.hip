@@ -53,6 +53,7 @@ struct ostft_ctx {
     hipStream_t stream = nullptr;  // internal: table builds
     std::mutex mu;                 // guards the table caches and `stream`
     std::map<std::pair<int64_t, int64_t>, float2*> twiddles;  // (m, count) -> W_m^j, j < count
+    std::map<std::pair<int64_t, int64_t>, double2*> twiddles64;
     std::map<std::tuple<int, int64_t, uint32_t, int>, float*> windows;  // (kind, N, sigma bits, exact)
     std::map<std::tuple<const float*, int, int>, void*> mfma_tables;  // (window table, log_m, format)
     std::mutex lanes_mu;
@@ -196,19 +197,21 @@ int not_prepared(ostft_ctx* ctx, const char* what)
 }
 
 // W_m^j for j < count, generated once and kept (with `noalloc`: looked up only).
-float2* get_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc = false)
+template <typename T2>
+T2* get_table(ostft_ctx* ctx, std::map<std::pair<int64_t, int64_t>, T2*>& tables, int64_t m, int64_t count, int* rc,
+              bool noalloc)
 {
     std::lock_guard<std::mutex> lk(ctx->mu);
     const auto key = std::make_pair(m, count);
-    auto it = ctx->twiddles.find(key);
-    if (it != ctx->twiddles.end())
+    auto it = tables.find(key);
+    if (it != tables.end())
         return it->second;
     if (noalloc) {
         *rc = not_prepared(ctx, "a twiddle table");
         return nullptr;
     }
-    float2* t = nullptr;
-    hipError_t e = hipMalloc(&t, sizeof(float2) * (size_t)count);
+    T2* t = nullptr;
+    hipError_t e = hipMalloc(&t, sizeof(T2) * (size_t)count);
     if (e == hipSuccess)
         e = ostft::launch_twiddle_table(t, m, count, ctx->stream);
     if (e == hipSuccess)
@@ -219,8 +222,13 @@ float2* get_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noa
         *rc = hip_fail(ctx, e, "twiddle table");
         return nullptr;
     }
-    ctx->twiddles[key] = t;
+    tables[key] = t;
     return t;
+}
+
+float2* get_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc = false)
+{
+    return get_table(ctx, ctx->twiddles, m, count, rc, noalloc);
 }
 
 // Window coefficients exactly as the reference computes them on the CPU
@@ -352,6 +360,10 @@ namespace ostft {
 float2* ctx_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc)
 {
     return get_twiddles(ctx, m, count, rc, noalloc);
+}
+double2* ctx_twiddles64(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc)
+{
+    return get_table(ctx, ctx->twiddles64, m, count, rc, noalloc);
 }
 bool ctx_has_twiddles(ostft_ctx* ctx, int64_t m, int64_t count)
 {
@@ -621,6 +633,8 @@ void ostft_destroy(ostft_ctx* ctx)
         DeviceGuard dg(ctx->device);
         (void)hipDeviceSynchronize();
         for (auto& kv : ctx->twiddles)
+            (void)hipFree(kv.second);
+        for (auto& kv : ctx->twiddles64)
             (void)hipFree(kv.second);
         for (auto& kv : ctx->windows)
             (void)hipFree(kv.second);

@@ -105,8 +105,9 @@ hipError_t launch_batch(int log_m, int variant, const BatchClassArgs& b, uint32_
 hipError_t batch_class_info(int log_m, int variant, BatchClassInfo* info);
 
 // FP64 table generators (run once per table).
-// tw[j] = exp(-2 pi i j / m) for j < count (count <= m)
-hipError_t launch_twiddle_table(float2* tw, int64_t m, int64_t count, hipStream_t s);
+// tw[j] = exp(-2 pi i j / m) for j < count (count <= m), as float2 or double2
+template <typename T2>
+hipError_t launch_twiddle_table(T2* tw, int64_t m, int64_t count, hipStream_t s);
 // window formulas of OKL/kernel.okl:33-127 evaluated in FP64, rounded once
 hipError_t launch_window_table(float* w, int64_t n, int kind, float sigma, hipStream_t s);
 

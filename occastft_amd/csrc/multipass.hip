@@ -266,16 +266,22 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
 
 struct LastArgs {
     const float2* src;   // first pass output
-    const float2* tw_r;  // W_R1^j, j < R1
     const float2* tw_n;  // W_N^k, k < M
-    // W_M^(k 2^j), k < R0: the powers the twists take, side by side for the
-    // butterflies of a wave (gathered from W_N^k, they would fetch as many
-    // bytes again as the scratch values)
+    // W_M^(k 2^j), k < R0: the powers the first step's twists take (2^16: the only
+    // step's), side by side for the butterflies of a wave (gathered from W_N^k, they
+    // would fetch as many bytes again as the scratch values)
     const float2* tw_k[9];
+    const double2* tw_m;  // W_M^k, k < R0, and
+    const double2* tw_r;  // W_R1^j, j < R1/16: their products are the second step's
     float* out;
     uint64_t frame0, frames, out_limit;  // frames [frame0, frames); scratch row 0 = frame0
     int32_t combine, out_mode, dc;
 };
+
+__device__ __forceinline__ double2 cmul64(double2 a, double2 b)
+{
+    return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
+}
 
 // Last pass: C / 2 butterflies k and their mirrors R0 - k (0 and R0/2 are their
 // own) of one frame, R points each with twist W_M^k: a step of r1 = R/16 points
@@ -359,13 +365,20 @@ __global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4)
             __syncthreads();
             gather_step<C, r1, PAD, T, 2, 1>(v, rd);
         }
-        // second step, butterfly t + T u over 16 inputs: twist W_M^k W_R^(t + T u)
+        // second step, butterfly t + T u over 16 inputs: twist W_M^k W_R^(t + T u),
+        // it and its squares formed in FP64 and rounded once (products of two float
+        // tables: error 2.82 for 2.46e-7 at 2^17, power, noise; the powers read from
+        // tables of M/16 entries: the same error, 2^20 719 -> 729 us, here 713)
+        const double2 wk = a.tw_m[k];
         cfor<0, 2>([&](auto u) {
             constexpr int UU = decltype(u)::value;
             Twist<16> tu;
+            double2 w = cmul64(wk, a.tw_r[t + T * UU]);
             cfor<0, 4>([&](auto l) {
-                constexpr uint32_t J = 3 - decltype(l)::value;
-                tu.base[decltype(l)::value] = cmul(a.tw_k[J][k], a.tw_r[(t + T * UU) << J]);
+                constexpr int L = 3 - decltype(l)::value;  // base[L] = w^(8 >> L)
+                tu.base[L] = make_float2((float)w.x, (float)w.y);
+                if constexpr (L > 0)
+                    w = cmul64(w, w);
             });
             twisted_dft<16, UU, 2, true>(v, tu);
         });
@@ -540,25 +553,31 @@ namespace {
 // `noalloc` a table that is not resident yet is an error instead of being
 // built.
 struct PassTables {
-    const float2 *r0, *r1, *k[9] = {};
+    const float2 *r0, *k[9] = {};
+    const double2 *m = nullptr, *r = nullptr;
 };
+
+// the powers W_M^(k 2^j) that the last pass reads start with this j
+int first_power(int log_m) { return log_m > 15 ? 4 : 0; }
 
 int pass_tables(ostft_ctx* ctx, int log_m, bool noalloc, PassTables* t)
 {
     int rc = OSTFT_OK;
-    const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
-    t->r1 = nullptr;
-    if ((t->r0 = ctx_twiddles(ctx, MP_R0, MP_R0, &rc, noalloc)))
-        t->r1 = ctx_twiddles(ctx, R1, R1, &rc, noalloc);
-    for (int j = 0; rc == OSTFT_OK && j < log_m - MP_LOG_R0; ++j)
+    t->r0 = ctx_twiddles(ctx, MP_R0, MP_R0, &rc, noalloc);
+    for (int j = first_power(log_m); rc == OSTFT_OK && j < log_m - MP_LOG_R0; ++j)
         t->k[j] = ctx_twiddles(ctx, (int64_t)1 << (log_m - j), MP_R0, &rc, noalloc);
+    if (rc == OSTFT_OK && first_power(log_m) > 0) {
+        const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
+        if ((t->m = ctx_twiddles64(ctx, (int64_t)1 << log_m, MP_R0, &rc, noalloc)))
+            t->r = ctx_twiddles64(ctx, R1, R1 / 16, &rc, noalloc);
+    }
     return rc;
 }
 
-bool tables_resident(ostft_ctx* ctx, int log_m)
+// those of window 2^16
+bool wide_tables_resident(ostft_ctx* ctx, int log_m)
 {
-    const int64_t R1 = (int64_t)1 << (log_m - MP_LOG_R0);
-    bool all = ctx_has_twiddles(ctx, MP_R0, MP_R0) && ctx_has_twiddles(ctx, R1, R1);
+    bool all = ctx_has_twiddles(ctx, MP_R0, MP_R0);
     for (int j = 0; all && j < log_m - MP_LOG_R0; ++j)
         all = ctx_has_twiddles(ctx, (int64_t)1 << (log_m - j), MP_R0);
     return all;
@@ -625,7 +644,8 @@ int run_chunks(ostft_ctx* ctx, int log_m, const FusedArgs& a, const PassTables& 
     p.tw_r = t.r0;
 
     LastArgs la;
-    la.tw_r = t.r1;
+    la.tw_m = t.m;
+    la.tw_r = t.r;
     la.tw_n = a.tw_n;
     std::copy(std::begin(t.k), std::end(t.k), la.tw_k);
     la.out = a.out;
@@ -715,7 +735,7 @@ int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
             // a captured call takes the passes with a buffer of its own, and tables
             // that are there (none can be built under capture)
             if (room && capture.on)
-                room = tables_resident(ctx, log_m) && sc.hold(capture, s, a.frames << log_m);
+                room = wide_tables_resident(ctx, log_m) && sc.hold(capture, s, a.frames << log_m);
         }
         if (room)
             return run_multipass(ctx, log_m, a, s);
@@ -728,7 +748,7 @@ int run_wide(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 // 20 23.5 / 17.4, 40 23.8 / 20.4.
 int run_wide_noalloc(ostft_ctx* ctx, int log_m, const FusedArgs& a, hipStream_t s)
 {
-    if (wide_in_passes(a) && tables_resident(ctx, log_m)) {
+    if (wide_in_passes(a) && wide_tables_resident(ctx, log_m)) {
         const int rc = run_multipass(ctx, log_m, a, s, true);
         if (rc != OSTFT_ERR_NOT_PREPARED)
             return rc;

@@ -48,6 +48,7 @@ struct Scratch {
 // W_m^j, j < count; with `noalloc` only a table already resident (else null
 // and OSTFT_ERR_NOT_PREPARED in *rc)
 float2* ctx_twiddles(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc = false);
+double2* ctx_twiddles64(ostft_ctx* ctx, int64_t m, int64_t count, int* rc, bool noalloc = false);
 bool ctx_has_twiddles(ostft_ctx* ctx, int64_t m, int64_t count);  // that table is resident
 Scratch& ctx_scratch(ostft_ctx* ctx);
 std::mutex& ctx_scratch_mutex(ostft_ctx* ctx);  // held while a call queues its scratch launches

@@ -1,28 +1,33 @@
 // tables.hip -- FP64 generators for the twiddle table and the exact window table.
 //
-// FP64 is used on the GPU only here.  Tables are built once per (size, kind)
-// and kept resident by the context.
+// Tables are built once per (size, kind) and kept resident by the context.
 #include "engine.hpp"
 
 namespace ostft {
 
 // tw[j] = exp(-2 pi i j / M) for j < count: sincospi of the exact rational -2j/M.
-__global__ void twiddle_kernel(float2* tw, int64_t m, int64_t count)
+template <typename T2>
+__global__ void twiddle_kernel(T2* tw, int64_t m, int64_t count)
 {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= count)
         return;
     double s, c;
     sincospi(-2.0 * (double)j / (double)m, &s, &c);
-    tw[j] = make_float2((float)c, (float)s);
+    using T = decltype(tw[j].x);
+    tw[j].x = (T)c;
+    tw[j].y = (T)s;
 }
 
-hipError_t launch_twiddle_table(float2* tw, int64_t m, int64_t count, hipStream_t s)
+template <typename T2>
+hipError_t launch_twiddle_table(T2* tw, int64_t m, int64_t count, hipStream_t s)
 {
     const int64_t blocks = (count + 255) / 256;
-    hipLaunchKernelGGL(twiddle_kernel, dim3((uint32_t)blocks), dim3(256), 0, s, tw, m, count);
+    hipLaunchKernelGGL(twiddle_kernel<T2>, dim3((uint32_t)blocks), dim3(256), 0, s, tw, m, count);
     return hipGetLastError();
 }
+template hipError_t launch_twiddle_table(float2* tw, int64_t m, int64_t count, hipStream_t s);
+template hipError_t launch_twiddle_table(double2* tw, int64_t m, int64_t count, hipStream_t s);
 
 constexpr double kPi = 3.14159265358979323846;
 
