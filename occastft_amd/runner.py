@@ -201,11 +201,11 @@ class Runner:
         for x, p, _ in jobs:
             if x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
                 raise ValueError("inputs must be contiguous float32 tensors on the GPU")
-            if not isinstance(p, N.Params):
-                raise TypeError(f"params must be Params, not {type(p).__name__}")
             ptrs.append(x.data_ptr())
             sizes.append(x.numel())
-            params.append(bytes(p))
+            params.append(p)
+        if set(map(type, params)) != {N.Params} and not all(isinstance(p, N.Params) for p in params):
+            raise TypeError("the params of every job must be Params")
         dev = x.device
         table = np.zeros(count, dtype=_JOB)
         table["in_ptr"] = ptrs
