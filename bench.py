@@ -665,7 +665,7 @@ def bench_batch(args, runner):
         for e in BATCH_EXPS:
             go, p, g, stride, _ = batch_launcher(runner, x, form, e, out)
             # at least two: the batch path alternates two descriptor blocks,
-            # each with its own captured launches, made on first use
+            # allocated on first use
             for _ in range(max(2, args.warmup)):
                 go()
             torch.cuda.synchronize()
@@ -910,8 +910,7 @@ def bench_serve(args, runner):
     for e in SERVE_EXPS:
         c = runner.autotune_batch(e, SERVE_TUNE_SAMPLES, like=like)
         choices[str(1 << e)] = {"blocks_per_cu": c.blocks_per_cu, "shape": c.shape, "plan": c.plan}
-    # both descriptor blocks' captured launches (re-made after the autotuner
-    # changed a variant) before the timed launches
+    # both descriptor blocks before the timed launches
     go()
     go()
     torch.cuda.synchronize()

@@ -11,8 +11,8 @@
 // the stream, the GPU stood idle 35-50 us between two batches: 9 before the
 // copy, 9 for 200 KB, 17-33 after it.)  The launches are made one by one: replaying
 // them from a captured graph with a node for each of the ten window sizes took
-// longer for every mix, 58 against 35 us a batch of 24 requests of three sizes, 280
-// against 274 us one of 256 requests of ten.
+// longer for both mixes measured, 58 against 35 us a batch of 24 requests of three
+// sizes, 280 against 257-274 us one of 256 requests of ten.
 //
 // Requests of windows >= 2^16 (one kernel or two passes) and requests of the matrix-core
 // form run after the tile-queue launches, one request at a time, on the same

@@ -29,10 +29,11 @@
 // compiled out the passes took within 10% of their time.  Against the form before
 // (16 values a thread, samples and scratch staged through LDS on their way in
 // and out, 2 to 3 exchanges, VALU issue 41-72% of the time), 2^27 samples:
-// window 2^18, overlap 0, default layout 594 -> 507 us (2.15 GB moved, 4.2 TB/s; a
-// plain copy of 2 GiB runs at 4.9); 2^20, 75%, power 2050 -> 1590 us; 2^26
-// samples, 75%, default layout: 2^17 853 -> 839, 2^18 987 -> 878, 2^19 1040 -> 903,
-// 2^20 1239 -> 961 us; one frame: 20-26 -> 15-20 us.
+// window 2^18, overlap 0, default layout 594 -> 507 us, with two chunks at a time
+// (below) 477 (2.15 GB moved, 4.5 TB/s; a plain copy of 2 GiB runs at 4.9); 2^20, 75%,
+// power 2050 -> 1590 -> 1388 us; 2^26 samples, 75%, default layout: 2^17 853 -> 839
+// -> 780, 2^18 987 -> 878 -> 821, 2^19 1040 -> 903 -> 858, 2^20 1239 -> 961 -> 908 us;
+// one frame: 20-26 -> 15-20 us.
 #include "../../include/occastft_hip.h"
 
 #include <algorithm>

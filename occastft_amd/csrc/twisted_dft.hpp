@@ -10,6 +10,10 @@
 // (level LEN uses w^(R/LEN) W_LEN^q).  A radix-32 pass with a twist is then
 // 480 FMAs and 11 products by constants, against 456 instructions for the
 // transform, 124 for its 31 input products and 104 to form the powers.
+// Butterflies of fused multiply-adds are known from the literature on FFTs for such
+// machines (E. Linzer and E. Feig, IEEE Trans. Signal Processing 41, 1993; S.
+// Goedecker, SIAM J. Sci. Comput. 18, 1997); a - c b is taken as 2 a - (a + c b), which
+// needs no ratio of the twiddle's parts.
 #pragma once
 
 #include "fft_device.hpp"
